@@ -520,6 +520,386 @@ __global__ void __launch_bounds__(256) recv_pre_wave_kernel(PreParams p) {
    }
 }
 
+// ------------------------------------------------------------------ cell form
+//
+// Sparse source into a target t times finer along x and y with one data patch
+// per source feature (the reconstruction of an LCA column).  The t target
+// columns of one cell (first column congruent to the patch starts modulo t)
+// are covered by the same source columns, so the cw*nf targets of one thread
+// (cw columns of a cell, all features) walk the same entries of the active
+// list: per covering source row one contiguous run, read from the caches a few
+// entries ahead, each entry feeding V = cw*nf sums with one LDS read of V
+// consecutive weights.  A workgroup owns one batch element and one residue of
+// the target rows modulo t (and one of t/cw column groups), which needs only
+// the weight rows of one class, 1/t of the weights: they stay in LDS, feature
+// by feature, an odd number of V-wide pieces apart, so that the lanes' reads at
+// unrelated features spread over the banks.  Waves take 64 (row, cell) items at
+// a time from a counter in LDS.  Each target adds the terms of
+// recv_pre_gather_kernel in its order: the row table in order, source columns
+// ascending, entries ascending.
+//
+// Lanes of a wave walk lists of different lengths (the activity follows the
+// image), so the items of a workgroup are first sorted by their number of
+// entries (a counting sort over 256 lengths, longest first): a wave's lanes
+// then end together, and the longest lists start first.  A lane moves on to
+// its next run by itself; the entries of its next batch are in flight while
+// the current one is added.
+//
+// Bound: the lanes' list reads (64 unrelated cache lines per load: reading the
+// entries in 16-byte pairs instead of one by one halved that), then the vector
+// instructions (about 18 per entry for four targets) and the weight reads from
+// LDS.  Measured against recv_pre_lds_kernel, which stages the lists in LDS
+// between barriers: 64 images, 32x32x512 -> 128x128x1, 16x16 patches, 44,776
+// actives per image, 1368 -> 317 us; one image, 64x32x24 -> 128x64x1, 18x18
+// patches, 715 -> 79 us.
+struct CellPlan {
+   int t, cw, qx, qy; // target cells per source cell; columns per thread; covering columns / rows
+   int fstride;       // LDS floats of one feature: V * (qx*qy | 1)
+   int splits;        // workgroups per (batch element, class)
+   float invNf, invT; // 1 / pre.nf, 1 / t
+};
+
+// V consecutive LDS values at byte offset o from wl, a multiple of 4*V.
+template <int V>
+__device__ __forceinline__ void cell_weights(const float *wl, uint32_t o, float (&w)[V]) {
+   const char *p = reinterpret_cast<const char *>(wl) + o;
+   if (V % 4 == 0) {
+#pragma unroll
+      for (int v = 0; v < V; v += 4) {
+         float4 const x = *reinterpret_cast<const float4 *>(p + 4 * v);
+         w[v]           = x.x;
+         w[v + 1]       = x.y;
+         w[v + 2]       = x.z;
+         w[v + 3]       = x.w;
+      }
+   }
+   else if (V % 2 == 0) {
+#pragma unroll
+      for (int v = 0; v < V; v += 2) {
+         float2 const x = *reinterpret_cast<const float2 *>(p + 4 * v);
+         w[v]           = x.x;
+         w[v + 1]       = x.y;
+      }
+   }
+   else {
+#pragma unroll
+      for (int v = 0; v < V; v++) {
+         w[v] = *reinterpret_cast<const float *>(p + 4 * v);
+      }
+   }
+}
+
+// four words on an 8-byte boundary
+typedef uint32_t uint4u __attribute__((ext_vector_type(4), aligned(8)));
+
+constexpr int kCellItems   = 2;   // items per thread sorted together
+constexpr int kCellBuckets = 256; // list lengths told apart by the sort
+
+template <int V, bool EXACT>
+__global__ void __launch_bounds__(1024) recv_pre_cell_kernel(PreParams p, CellPlan c) {
+   extern __shared__ float smem[];
+   float *wl       = smem;
+   uint32_t *hist  = reinterpret_cast<uint32_t *>(smem + p.pre.nf * c.fstride); // [kCellBuckets]
+   uint32_t *ctl   = hist + kCellBuckets;                                       // next wave, longest list
+   uint16_t *order = reinterpret_cast<uint16_t *>(ctl + 2);                     // [kCellItems * blockDim.x]
+   int const tid   = threadIdx.x;
+   int const lane  = tid % kWave;
+   int const t     = c.t;
+   int const nf    = p.post.nf;
+   int const nfPre = p.pre.nf;
+   int const nxExt = p.pre.nxExt();
+   int const rho   = blockIdx.y % t;        // target rows rho, rho + t, ...
+   int const dx0   = blockIdx.y / t * c.cw; // this workgroup's columns of a cell
+   int const b     = blockIdx.z;
+   // first column of cell 0 (at most 0) and the weight-row class of this residue
+   // (from the first covered column and row; without one there is nothing to add)
+   int X0 = 0, cls = 0;
+   for (int X = 0; X < p.post.nx; X++) {
+      int const ci = p.colPtr[X];
+      if (p.colPtr[X + 1] > ci) {
+         X0 = (X - p.colWx[ci] % t + t) % t;
+         X0 -= X0 > 0 ? t : 0;
+         break;
+      }
+   }
+   for (int Y = rho; Y < p.post.ny; Y += t) {
+      int const ri = p.rowPtr[Y * p.nyp];
+      if (p.rowPtr[(Y + 1) * p.nyp] > ri) {
+         cls = p.rowWy[ri] % t;
+         break;
+      }
+   }
+   int const cells = (p.post.nx - X0 + t - 1) / t;
+   int const rows  = (p.post.ny - rho + t - 1) / t;
+   int const items = rows * cells;
+   int const waves = (items + kWave - 1) / kWave;
+   int const first = (int)((long long)waves * blockIdx.x / c.splits) * kWave;
+   int const last  = min((int)((long long)waves * (blockIdx.x + 1) / c.splits) * kWave, items);
+   {
+      // weights [f][jy][jx][V]: patch rows cls + t*jy, columns dx0 + t*jx ..
+      int const q         = c.qx * c.qy;
+      int const patchSize = p.nxp * p.nyp * nf;
+      for (int i = tid; i < nfPre * q; i += blockDim.x) {
+         int const f      = i / q;
+         int const j      = i - f * q;
+         int const jy     = j / c.qx;
+         int const jx     = j - jy * c.qx;
+         float const *src = p.W + (size_t)f * patchSize + ((cls + t * jy) * p.nxp + dx0 + t * jx) * nf;
+         float *dst       = wl + f * c.fstride + j * V;
+#pragma unroll
+         for (int v = 0; v < V; v++) {
+            dst[v] = src[v];
+         }
+      }
+   }
+   const uint32_t *ps = p.posStart + (size_t)b * ((size_t)nxExt * p.pre.nyExt() + 1);
+   const char *ent    = reinterpret_cast<const char *>(p.active + (size_t)b * p.pre.numExt());
+   float *gb          = p.gsyn + (size_t)b * p.post.numRes();
+   uint32_t const lastPair = (uint32_t)p.pre.numExt() - 2; // numExt is even
+   uint32_t const lastOff = (uint32_t)(nfPre * c.fstride - V) * 4;
+   int const rowF     = p.post.nx * nf;
+   int const qV       = nfPre * c.fstride + V; // LDS step back from one source column to the next
+   // target row, first column and covering rows / columns of an item
+   struct Item {
+      int Y, Xs, c0, ncol, r0, r1;
+   };
+   auto item_of = [&](int item) {
+      Item it;
+      int const m  = item / cells;
+      it.Y         = rho + t * m;
+      it.Xs        = X0 + t * (item - m * cells) + dx0;
+      int const Xv = max(it.Xs, 0); // the first column inside the target
+      it.c0 = it.ncol = it.r0 = it.r1 = 0;
+      if (it.Xs + c.cw > 0 && Xv < p.post.nx) {
+         it.c0   = p.colPtr[Xv];
+         it.ncol = p.colPtr[Xv + 1] - it.c0;
+         if (it.ncol > 0) {
+            it.r0 = p.rowPtr[it.Y * p.nyp];
+            it.r1 = p.rowPtr[(it.Y + 1) * p.nyp];
+         }
+      }
+      return it;
+   };
+   for (int base = first; base < last; base += kCellItems * blockDim.x) {
+      int const n     = min((int)(kCellItems * blockDim.x), last - base);
+      bool const sort = n > kWave;
+      __syncthreads(); // the staged weights; the order of the items before is read
+      if (tid < 2) {
+         ctl[tid] = 0;
+      }
+      if (sort) {
+         for (int i = tid; i < kCellBuckets; i += blockDim.x) {
+            hist[i] = 0;
+         }
+         uint32_t len[kCellItems];
+         uint32_t longest = 0;
+#pragma unroll
+         for (int u = 0; u < kCellItems; u++) {
+            int const j = tid + u * blockDim.x;
+            len[u]      = 0;
+            if (j < n) {
+               Item const it = item_of(base + j);
+               int const xe0 = it.ncol > 0 ? p.colXe[it.c0] : 0;
+               for (int ri = it.r0; ri < it.r1; ri++) {
+                  int const pos = p.rowYe[ri] * nxExt + xe0;
+                  len[u] += ps[pos + it.ncol] - ps[pos];
+               }
+            }
+            longest = max(longest, len[u]);
+         }
+         __syncthreads();
+         atomicMax(&ctl[1], longest);
+         __syncthreads();
+         float const scale = (float)(kCellBuckets - 1) / (float)max(ctl[1], 1u);
+         uint32_t rank[kCellItems];
+         int bucket[kCellItems];
+#pragma unroll
+         for (int u = 0; u < kCellItems; u++) {
+            bucket[u] = kCellBuckets - 1 - min(kCellBuckets - 1, (int)((float)len[u] * scale));
+            rank[u]   = tid + u * (int)blockDim.x < n ? atomicAdd(&hist[bucket[u]], 1u) : 0u;
+         }
+         __syncthreads();
+         if (tid < kWave) { // exclusive scan of the buckets, four per lane
+            constexpr int PER = kCellBuckets / kWave;
+            uint32_t h[PER];
+            uint32_t sum = 0;
+#pragma unroll
+            for (int u = 0; u < PER; u++) {
+               h[u] = sum;
+               sum += hist[PER * lane + u];
+            }
+            uint32_t incl = sum;
+#pragma unroll
+            for (int off = 1; off < kWave; off <<= 1) {
+               uint32_t const v = __shfl_up(incl, off, kWave);
+               incl += lane >= off ? v : 0u;
+            }
+#pragma unroll
+            for (int u = 0; u < PER; u++) {
+               hist[PER * lane + u] = h[u] + incl - sum;
+            }
+         }
+         __syncthreads();
+#pragma unroll
+         for (int u = 0; u < kCellItems; u++) {
+            int const j = tid + u * blockDim.x;
+            if (j < n) {
+               order[hist[bucket[u]] + rank[u]] = (uint16_t)j;
+            }
+         }
+      }
+      __syncthreads();
+      for (;;) {
+         uint32_t wi = 0;
+         if (lane == 0) {
+            wi = atomicAdd(&ctl[0], 1u);
+         }
+         wi = __builtin_amdgcn_readfirstlane(wi);
+         if ((int)wi * kWave >= n) {
+            break; // the whole wave
+         }
+         int const slot = (int)wi * kWave + lane;
+         if (slot < n) {
+            Item const it = item_of(base + (sort ? (int)order[slot] : slot));
+            float *grow   = gb + (size_t)it.Y * rowF;
+            float acc[V];
+#pragma unroll
+            for (int v = 0; v < V; v++) {
+               int const o = it.Xs * nf + v;
+               acc[v]      = (p.accumulate && o >= 0 && o < rowF) ? grow[o] : 0.0f;
+            }
+            int const xe0 = it.ncol > 0 ? p.colXe[it.c0] : 0;
+            int const jx0 = it.ncol > 0 ? (p.colWx[it.c0] - (max(it.Xs, 0) - it.Xs)) / t : 0;
+            // Runs of the covering rows, in table order: run ri holds entries
+            // [s, e) of the list; kex0 is the extended index of its first
+            // possible feature, w the LDS offset (bytes) of its weights.  The
+            // run after the current one is loaded a run ahead, its row number
+            // two runs ahead.
+            auto row_at  = [&](int ri) { return max(min(ri, it.r1 - 1), 0); };
+            int ri       = it.r0;
+            uint32_t nS  = 0, nE = 0;
+            int nPos     = 0, nWy = 0;
+            int ye2      = p.rowYe[row_at(ri)];
+            int wy2      = p.rowWy[row_at(ri)];
+            auto load_next = [&](int r) { // run r into nS.., row r + 1 into ye2, wy2
+               nPos = ye2 * nxExt + xe0;
+               nWy  = wy2;
+               nS   = ps[nPos];
+               nE   = ps[nPos + it.ncol];
+               ye2  = p.rowYe[row_at(r + 1)];
+               wy2  = p.rowWy[row_at(r + 1)];
+            };
+            uint32_t s = 0, e = 0, kex0 = 0;
+            int w = 0, skip = 0;
+            auto take_next = [&]() {
+               s    = nS & ~1u; // 16-byte pairs of entries
+               skip = nS & 1;
+               e    = nE;
+               kex0 = (uint32_t)nPos * (uint32_t)nfPre;
+               // (wy - cls) / t by the reciprocal, exact for these sizes
+               w = ((int)((float)(nWy - cls) * c.invT + 0.5f) * c.qx + jx0) * (V * 4);
+            };
+            constexpr int U = V <= 4 ? 8 : 4; // entries of a batch
+            uint4u en[U / 2];
+            auto fetch = [&]() {
+#pragma unroll
+               for (int u = 0; u < U; u += 2) {
+                  en[u / 2] = *reinterpret_cast<const uint4u *>(ent + min(s + u, lastPair) * 8u);
+               }
+            };
+            load_next(ri);
+            take_next();
+            load_next(ri + 1);
+            fetch();
+            while (ri < it.r1) {
+               int const left  = (int)(e - s);
+               int const left0 = skip ? 0 : left;
+               float wv[U][V], a[U];
+#pragma unroll
+               for (int u = 0; u < U; u++) {
+                  // feature f of source column xe0 + k: d = k*nfPre + f; an
+                  // entry past the run may hold anything: its read is clamped to
+                  // the staged weights
+                  uint32_t const d = en[u / 2][u % 2 * 2] - kex0;
+                  int const k      = (int)__builtin_fmaf((float)d, c.invNf, 0.5f * c.invNf);
+                  int const off    = (int)__umul24(d, c.fstride * 4) + w;
+                  cell_weights<V>(wl, min((uint32_t)(__mul24(k, -4 * qV) + off), lastOff), wv[u]);
+                  a[u] = __uint_as_float(en[u / 2][u % 2 * 2 + 1]) * p.dtf;
+               }
+               s += U;
+               skip = 0;
+               if (s >= e) {
+                  ri++;
+                  take_next();
+                  load_next(ri + 1);
+               }
+               fetch(); // in flight during this batch's sums
+#pragma unroll
+               for (int u = 0; u < U; u++) {
+                  if (u < (u == 0 ? left0 : left)) {
+#pragma unroll
+                     for (int v = 0; v < V; v++) {
+                        if (EXACT) {
+                           float const prod = a[u] * wv[u][v];
+                           acc[v]           = acc[v] + prod;
+                        }
+                        else {
+                           acc[v] = __builtin_fmaf(a[u], wv[u][v], acc[v]);
+                        }
+                     }
+                  }
+               }
+            }
+#pragma unroll
+            for (int v = 0; v < V; v++) {
+               int const o = it.Xs * nf + v;
+               if (o >= 0 && o < rowF) {
+                  grow[o] = acc[v];
+               }
+            }
+         }
+      }
+   }
+}
+
+// The cell form of a delivery, or t == 0 where it does not apply: a target t
+// times finer, one data patch per feature, patches of whole cells, and a class
+// of the weights that fits the LDS for some number of columns per thread.
+// Weights, buckets and control words; the sort's order takes up to 4 KB more.
+constexpr size_t kCellLdsMax = 155 * 1024;
+
+CellPlan cell_plan(const PreParams &p, size_t *lds) {
+   CellPlan c{};
+   int const t = p.pre.nx > 0 ? p.post.nx / p.pre.nx : 0;
+   if (!p.posStart || p.nKx != 1 || p.nKy != 1 || t < 1 || p.post.nx != t * p.pre.nx
+       || p.post.ny != t * p.pre.ny || p.nxp % t || p.nyp % t || t * t > 65535 || p.post.nbatch > 65535) {
+      return c;
+   }
+   c.qx = p.nxp / t;
+   c.qy = p.nyp / t;
+   // an entry's column comes from a float division, exact far below 2^22; its
+   // byte offset in the list is a 32-bit number; entries are read in pairs
+   if ((long long)c.qx * p.pre.nf > (1 << 20) || p.pre.numExt() >= (1 << 28) || p.pre.numExt() % 2) {
+      return c;
+   }
+   for (int cw = t; cw >= 1; cw--) {
+      int const V = cw * p.post.nf;
+      if (t % cw || (V != 1 && V != 2 && V != 3 && V != 4 && V != 6 && V != 8)) {
+         continue;
+      }
+      c.fstride = V * (c.qx * c.qy | 1);
+      *lds      = (size_t)p.pre.nf * c.fstride * sizeof(float) + (kCellBuckets + 2) * sizeof(uint32_t);
+      if (*lds <= kCellLdsMax) {
+         c.t     = t;
+         c.cw    = cw;
+         c.invNf = 1.0f / (float)p.pre.nf;
+         c.invT  = 1.0f / (float)t;
+         return c;
+      }
+   }
+   return c;
+}
+
 } // namespace
 } // namespace pvhip
 
@@ -581,6 +961,44 @@ int pvhip_recv_pre(const pvhip_recv_pre_args *a, pvhip_stream stream) {
          hipLaunchKernelGGL(recv_pre_wave_kernel<false>, grid, dim3(256), 0, s, p);
       }
       PVHIP_LAUNCHED("recv_pre_wave");
+      return PVHIP_OK;
+   }
+   // Cell form for a sparse source into a finer, narrow target (1368 -> 317 us
+   // and 715 -> 79 us against the LDS-staged form below, which keeps coarser
+   // targets, several data patches and weights too large for the LDS).
+   size_t cellLds      = 0;
+   CellPlan cp         = cell_plan(p, &cellLds);
+   if (cp.t > 0) {
+      int const V       = cp.cw * p.post.nf;
+      int const classes = cp.t * (cp.t / cp.cw);
+      // (row, cell) items of one class in waves of 64; enough workgroups for
+      // about two per CU, or one where its weights take more than half the LDS
+      int const waves   = (((p.post.ny + cp.t - 1) / cp.t) * (p.pre.nx + 1) + kWave - 1) / kWave;
+      long long const g = (long long)p.post.nbatch * classes;
+      int const want    = cellLds > 80 * 1024 ? 256 : 512;
+      cp.splits         = (int)std::min<long long>(waves, std::max<long long>(1, (want + g - 1) / g));
+      int const threads = kWave * std::min(16, (waves + cp.splits - 1) / cp.splits);
+      cellLds += (size_t)threads * kCellItems * sizeof(uint16_t);
+      dim3 grid(cp.splits, classes, p.post.nbatch);
+#define PVHIP_CELL(VV)                                                                                   \
+   case VV:                                                                                              \
+      if (exact) {                                                                                       \
+         hipLaunchKernelGGL((recv_pre_cell_kernel<VV, true>), grid, dim3(threads), cellLds, s, p, cp);    \
+      }                                                                                                  \
+      else {                                                                                             \
+         hipLaunchKernelGGL((recv_pre_cell_kernel<VV, false>), grid, dim3(threads), cellLds, s, p, cp);   \
+      }                                                                                                  \
+      break;
+      switch (V) {
+         PVHIP_CELL(1)
+         PVHIP_CELL(2)
+         PVHIP_CELL(3)
+         PVHIP_CELL(4)
+         PVHIP_CELL(6)
+         PVHIP_CELL(8)
+      }
+#undef PVHIP_CELL
+      PVHIP_LAUNCHED("recv_pre_cell");
       return PVHIP_OK;
    }
    // LDS-staged form for sparse pre layers whose post features fit one workgroup.

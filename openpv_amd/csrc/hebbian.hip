@@ -90,8 +90,19 @@ __global__ void __launch_bounds__(256) hebbian_exact_kernel(HebbParams p) {
 // N = patch items (ky, kx, f'), K = batch x pre extended positions.  P is the
 // post activity with every value outside the post restricted region read as
 // 0, which is the reference's shrunken patch (pvhost_hebbian_windows checks
-// the geometry).  Counts (normalizeDw) are the same correlation of the
-// indicators a_pre != 0 and "inside the restricted region".
+// the geometry).
+//
+// Counts (normalizeDw): an active pre neuron counts for the items of its
+// window inside the post restricted region, an interval of window rows times
+// an interval of window columns.  Each active neuron is added to the corners of
+// its rectangle in an integer difference array D[ky][kx][f], whose
+// two-dimensional prefix sums are the counts.  Neurons whose whole window is
+// inside, all but a few rows and columns of the layer, add to (0, 0) only: the
+// workgroups of the first item block count them as they stage the activity.
+// hebbian_border_kernel adds the others.  (Counted by a second correlation, of
+// the indicators, they took 710 us beside the 370 us of dW for
+// 8 x 128x128x1024 -> 16x16 in BF16, and 96 beside 65 us for
+// 7 x 45x37x200 -> 8x8x3 in FP32.)
 //
 // Workgroup: 64 features x 256 items, 4 waves; wave w owns items
 // 64w .. 64w+63 (4 MFMA column blocks) for all 64 features (4 row blocks).
@@ -116,6 +127,8 @@ struct HebbMfma {
    int rowsPerChunk;
    const float *preData, *postData;
    float *part; // [chunks][nK][N]
+   int *diff;   // [nyp][nxp][nK] differences of the activation counts, or NULL
+   int xA, xB, yA, yB; // pre extended columns and rows whose whole window is inside
 };
 
 template <typename T>
@@ -167,8 +180,8 @@ constexpr int HAREG = 32;
 constexpr int HBR = 4;
 constexpr int HBX = 3;
 
-template <typename T, bool COUNT>
-__global__ void __launch_bounds__(256) hebbian_mfma_kernel(HebbMfma h) {
+template <typename T>
+__global__ void __launch_bounds__(256, 2) hebbian_mfma_kernel(HebbMfma h) {
    extern __shared__ float smem[];
    int const copies = sizeof(T) == 2 ? 2 : 1;
    int const nbrow  = h.nyp * h.nfp * h.sx; // B rows (ring slot, feature, phase)
@@ -222,9 +235,6 @@ __global__ void __launch_bounds__(256) hebbian_mfma_kernel(HebbMfma h) {
       float v      = 0.0f;
       if (xe < nxExt && f0 + m < h.nK) {
          v = h.preData[(((size_t)b * nyExt + ye) * nxExt + xe) * h.pre.nf + f0 + m];
-         if (COUNT) {
-            v = v != 0.0f ? 1.0f : 0.0f;
-         }
       }
       return v;
    };
@@ -257,8 +267,7 @@ __global__ void __launch_bounds__(256) hebbian_mfma_kernel(HebbMfma h) {
       int const px = h.sx * (xq + h.qx0) + ph;
       bool const in = py >= h.post.up && py < h.post.up + h.post.ny && px >= h.post.lt
                       && px < h.post.lt + h.post.nx;
-      return in ? (COUNT ? 1.0f : h.postData[(size_t)b * h.post.numExt() + ((size_t)py * nxExtP + px) * h.post.nf + fp])
-                : 0.0f;
+      return in ? h.postData[(size_t)b * h.post.numExt() + ((size_t)py * nxExtP + px) * h.post.nf + fp] : 0.0f;
    };
    auto b_put = [&](int py, int fp, int ph, int xq, float v) {
       int const idx = ring(py) * rowB + (fp * h.sx + ph) * h.lq + xq;
@@ -293,14 +302,15 @@ __global__ void __launch_bounds__(256) hebbian_mfma_kernel(HebbMfma h) {
          float v      = 0.0f;
          if (fok && xe < nxExt) {
             v = base[(size_t)(256 / HMT) * u * h.pre.nf];
-            if (COUNT) {
-               v = v != 0.0f ? 1.0f : 0.0f;
-            }
          }
          va[u] = v;
       }
    };
+   bool const counting = h.diff != nullptr && blockIdx.y == 0;
+   int active          = 0; // active neurons of feature f0 + am with a whole window
    auto stage = [&](int row) {
+      int const ye     = row % nyExt;
+      bool const whole = counting && ye >= h.yA && ye < h.yB;
 #pragma unroll
       for (int u = 0; u < HAREG; u++) {
          int const i = tid + 256 * u;
@@ -308,8 +318,21 @@ __global__ void __launch_bounds__(256) hebbian_mfma_kernel(HebbMfma h) {
             al[(i % HMT) * h.apitch + i / HMT] = hcvt<T>(va[u]);
          }
       }
+      if (whole) {
+#pragma unroll
+         for (int u = 0; u < HAREG; u++) { // pre column wave + 4*u, the same for the whole wave
+            int const xe = wave + (256 / HMT) * u;
+            if (xe >= h.xA && xe < h.xB) {
+               active += va[u] != 0.0f ? 1 : 0;
+            }
+         }
+      }
       for (int i = tid + 256 * HAREG; i < aItems; i += 256) {
-         al[(i % HMT) * h.apitch + i / HMT] = hcvt<T>(a_val(row, i));
+         float const v = a_val(row, i);
+         al[(i % HMT) * h.apitch + i / HMT] = hcvt<T>(v);
+         if (whole && i / HMT >= h.xA && i / HMT < h.xB) {
+            active += v != 0.0f ? 1 : 0;
+         }
       }
       int pyA, pyB;
       new_rows(row, pyA, pyB);
@@ -392,6 +415,9 @@ __global__ void __launch_bounds__(256) hebbian_mfma_kernel(HebbMfma h) {
          }
       }
    }
+   if (active > 0) { // va is 0 past the last feature
+      atomicAdd(h.diff + f0 + am, active);
+   }
    // D[4g+i][r]: feature f0 + mb*16 + 4g + i, item of lane r in block nb
    float *out = h.part + (size_t)chunk * h.nK * h.N;
 #pragma unroll
@@ -410,31 +436,139 @@ __global__ void __launch_bounds__(256) hebbian_mfma_kernel(HebbMfma h) {
    }
 }
 
-// dw[i] += dWMax * sum_c part[c][i] (chunks in order); counts[i] += sum_c cpart[c][i].
-__global__ void __launch_bounds__(256) hebbian_reduce_kernel(
-      const float *part, const float *cpart, int chunks, size_t n, float dwMax, float *dw,
-      int64_t *counts) {
-   size_t const i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-   if (i >= n) {
+// Counts of the pre neurons whose window is cut by the edge of the post
+// restricted region: one thread per feature and segment of up to kBorderRun
+// neurons with the same rectangle -- a run of whole rows of a cut column, a run
+// of whole columns of a cut row, or one neuron where both are cut.
+constexpr int kBorderRun = 32;
+
+__global__ void __launch_bounds__(256) hebbian_border_kernel(HebbMfma h) {
+   int const f     = blockIdx.y * kWave + threadIdx.x % kWave;
+   int seg         = blockIdx.x * (256 / kWave) + threadIdx.x / kWave;
+   int const nxExt = h.pre.nxExt();
+   int const nyExt = h.pre.nyExt();
+   int const nbx   = nxExt - (h.xB - h.xA); // cut columns, rows
+   int const nby   = nyExt - (h.yB - h.yA);
+   int const runsY = (h.yB - h.yA + kBorderRun - 1) / kBorderRun;
+   int const runsX = (h.xB - h.xA + kBorderRun - 1) / kBorderRun;
+   int const per   = nbx * runsY + nby * runsX + nby * nbx; // segments of a batch element
+   int const b     = seg / per;
+   if (b >= h.pre.nbatch || f >= h.nK) {
       return;
    }
-   float s = 0.0f;
-   for (int c = 0; c < chunks; c++) {
-      s = s + part[(size_t)c * n + i];
+   seg -= b * per;
+   auto cut_x = [&](int i) { return i < h.xA ? i : i - h.xA + h.xB; };
+   auto cut_y = [&](int i) { return i < h.yA ? i : i - h.yA + h.yB; };
+   int xe, ye, n, step = 0; // first neuron, their number, positions from one to the next
+   if (seg < nbx * runsY) {
+      xe   = cut_x(seg / runsY);
+      ye   = h.yA + seg % runsY * kBorderRun;
+      n    = min(kBorderRun, h.yB - ye);
+      step = nxExt;
+   }
+   else if (seg < nbx * runsY + nby * runsX) {
+      seg -= nbx * runsY;
+      ye   = cut_y(seg / runsX);
+      xe   = h.xA + seg % runsX * kBorderRun;
+      n    = min(kBorderRun, h.xB - xe);
+      step = 1;
+   }
+   else {
+      seg -= nbx * runsY + nby * runsX;
+      ye = cut_y(seg / nbx);
+      xe = cut_x(seg % nbx);
+      n  = 1;
+   }
+   // rectangle [ya, yb) x [xa, xb) of window items inside the restricted region
+   int const sx = h.sx * (xe + h.qx0) + h.cx0;
+   int const sy = h.sy * ye + h.cy;
+   int const xa = max(0, min(h.nxp, h.post.lt - sx));
+   int const xb = max(0, min(h.nxp, h.post.lt + h.post.nx - sx));
+   int const ya = max(0, min(h.nyp, h.post.up - sy));
+   int const yb = max(0, min(h.nyp, h.post.up + h.post.ny - sy));
+   if (xa >= xb || ya >= yb) {
+      return;
+   }
+   float const *v = h.preData + (((size_t)b * nyExt + ye) * nxExt + xe) * h.nK + f;
+   int on         = 0;
+#pragma unroll 8
+   for (int i = 0; i < n; i++) {
+      on += v[(size_t)i * step * h.nK] != 0.0f ? 1 : 0;
+   }
+   if (on > 0) {
+      atomicAdd(h.diff + (ya * h.nxp + xa) * h.nK + f, on);
+      if (xb < h.nxp) {
+         atomicAdd(h.diff + (ya * h.nxp + xb) * h.nK + f, -on);
+      }
+      if (yb < h.nyp) {
+         atomicAdd(h.diff + (yb * h.nxp + xa) * h.nK + f, -on);
+         if (xb < h.nxp) {
+            atomicAdd(h.diff + (yb * h.nxp + xb) * h.nK + f, on);
+         }
+      }
+   }
+}
+
+// dw[f][n] += dWMax * sum_c part[c][f][n] (chunks in order, eight loads in
+// flight); counts[f][n] += the prefix sum of diff[..][..][f] at the item's
+// window row and column.  Grid (features, ceil(N / 256)).
+__global__ void __launch_bounds__(256) hebbian_reduce_kernel(
+      const float *part, const int *diff, int chunks, int N, int nyp, int nxp, int nfp, float dwMax, float *dw,
+      int64_t *counts) {
+   extern __shared__ int sums[]; // [nyp][nxp]
+   int const f    = blockIdx.x;
+   int const tid  = threadIdx.x;
+   if (counts) {
+      int const items = nyp * nxp;
+      for (int i = tid; i < items; i += 256) {
+         sums[i] = diff[(size_t)i * gridDim.x + f];
+      }
+      __syncthreads();
+      for (int y = tid; y < nyp; y += 256) {
+         for (int x = 1; x < nxp; x++) {
+            sums[y * nxp + x] += sums[y * nxp + x - 1];
+         }
+      }
+      __syncthreads();
+      for (int x = tid; x < nxp; x += 256) {
+         for (int y = 1; y < nyp; y++) {
+            sums[y * nxp + x] += sums[(y - 1) * nxp + x];
+         }
+      }
+      __syncthreads();
+   }
+   int const n = blockIdx.y * 256 + tid;
+   if (n >= N) {
+      return;
+   }
+   size_t const i      = (size_t)f * N + n;
+   size_t const stride = (size_t)gridDim.x * N;
+   float s             = 0.0f;
+   int c               = 0;
+   for (; c + 8 <= chunks; c += 8) {
+      float v[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) {
+         v[u] = part[(size_t)(c + u) * stride + i];
+      }
+#pragma unroll
+      for (int u = 0; u < 8; u++) {
+         s = s + v[u];
+      }
+   }
+   for (; c < chunks; c++) {
+      s = s + part[(size_t)c * stride + i];
    }
    dw[i] = dw[i] + dwMax * s;
    if (counts) {
-      float cs = 0.0f;
-      for (int c = 0; c < chunks; c++) {
-         cs = cs + cpart[(size_t)c * n + i];
-      }
-      counts[i] += (int64_t)cs;
+      counts[i] += sums[n / nfp];
    }
 }
 
 struct HebbPlan {
    int chunks, rowsPerChunk, kxPad, lq, apitch;
    size_t lds, partBytes;
+   size_t diffBytes; // difference array of the counts
 };
 
 HebbPlan hebb_plan(const pvhip_hebbian_args &a, bool bf) {
@@ -463,6 +597,7 @@ HebbPlan hebb_plan(const pvhip_hebbian_args &a, bool bf) {
    size_t cstr     = ((size_t)a.nyp * a.nfp * sx * pl.lq + 7) / 8 * 8;
    pl.lds          = ((size_t)copies * cstr + (size_t)HMT * pl.apitch) * esz;
    pl.partBytes    = (size_t)pl.chunks * nK * N * sizeof(float);
+   pl.diffBytes    = a.counts ? (size_t)nK * a.nyp * a.nxp * sizeof(int) : 0;
    return pl;
 }
 
@@ -491,11 +626,11 @@ int pvhip_hebbian_dw(const pvhip_hebbian_args *a, pvhip_stream stream) {
       PVHIP_REQUIRE(a->window_stride_x > 0 && a->window_stride_y > 0,
             "hebbian_dw: the MFMA forms need the window geometry (pvhost_hebbian_windows)");
       HebbPlan pl = hebb_plan(*a, bf);
-      size_t need = pl.partBytes * (a->counts ? 2 : 1);
+      size_t need = pl.partBytes + pl.diffBytes;
       PVHIP_REQUIRE(a->scratch && a->scratch_bytes >= need,
             "hebbian_dw: scratch of %zu bytes, %zu needed", a->scratch_bytes, need);
       PVHIP_REQUIRE(pl.lds <= 160 * 1024, "hebbian_dw: tile needs %zu bytes of LDS", pl.lds);
-      HebbMfma h;
+      HebbMfma h{};
       h.pre     = geo(a->pre);
       h.post    = geo(a->post);
       h.nxp     = a->nxp;
@@ -516,30 +651,48 @@ int pvhip_hebbian_dw(const pvhip_hebbian_args *a, pvhip_stream stream) {
       h.preData  = a->pre_data;
       h.postData = a->post_data;
       float *part  = static_cast<float *>(a->scratch);
-      float *cpart = a->counts ? part + pl.partBytes / sizeof(float) : nullptr;
       dim3 grid((h.nK + HMT - 1) / HMT, (h.N + HNT - 1) / HNT, pl.chunks);
       hipStream_t s = (hipStream_t)stream;
       h.part        = part;
+      h.diff        = a->counts ? reinterpret_cast<int *>(part + pl.partBytes / sizeof(float)) : nullptr;
+      if (h.diff) {
+         int st = pvhip_fill_zero(h.diff, pl.diffBytes, stream);
+         if (st) {
+            return st;
+         }
+         // whole windows: start >= lo and start + patch <= lo + n
+         auto whole = [](int start0, int stride, int lo, int n, int patch, int ext, int &first, int &end) {
+            int const a = lo - start0, z = lo + n - patch - start0;
+            first       = std::min(ext, a > 0 ? (a + stride - 1) / stride : 0);
+            end         = z < 0 ? 0 : std::min(ext, z / stride + 1);
+            if (end <= first) {
+               first = end = 0;
+            }
+         };
+         whole(a->window_start_x, h.sx, h.post.lt, h.post.nx, h.nxp, h.pre.nxExt(), h.xA, h.xB);
+         whole(a->window_start_y, h.sy, h.post.up, h.post.ny, h.nyp, h.pre.nyExt(), h.yA, h.yB);
+      }
       if (bf) {
-         hipLaunchKernelGGL((hebbian_mfma_kernel<__bf16, false>), grid, dim3(256), pl.lds, s, h);
+         hipLaunchKernelGGL(hebbian_mfma_kernel<__bf16>, grid, dim3(256), pl.lds, s, h);
       }
       else {
-         hipLaunchKernelGGL((hebbian_mfma_kernel<float, false>), grid, dim3(256), pl.lds, s, h);
+         hipLaunchKernelGGL(hebbian_mfma_kernel<float>, grid, dim3(256), pl.lds, s, h);
       }
       PVHIP_LAUNCHED("hebbian_mfma");
-      if (cpart) {
-         h.part = cpart;
-         if (bf) {
-            hipLaunchKernelGGL((hebbian_mfma_kernel<__bf16, true>), grid, dim3(256), pl.lds, s, h);
+      if (h.diff) {
+         long long const nbx = h.pre.nxExt() - (h.xB - h.xA), nby = h.pre.nyExt() - (h.yB - h.yA);
+         long long const segs = (nbx * ((h.yB - h.yA + kBorderRun - 1) / kBorderRun)
+                                 + nby * ((h.xB - h.xA + kBorderRun - 1) / kBorderRun) + nby * nbx)
+                                * h.pre.nbatch;
+         if (segs > 0) {
+            hipLaunchKernelGGL(hebbian_border_kernel, dim3((unsigned)((segs + 3) / 4), (h.nK + kWave - 1) / kWave),
+                  dim3(256), 0, s, h);
+            PVHIP_LAUNCHED("hebbian_border");
          }
-         else {
-            hipLaunchKernelGGL((hebbian_mfma_kernel<float, true>), grid, dim3(256), pl.lds, s, h);
-         }
-         PVHIP_LAUNCHED("hebbian_mfma_counts");
       }
-      size_t n = (size_t)h.nK * h.N;
-      hipLaunchKernelGGL(hebbian_reduce_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s,
-            part, cpart, pl.chunks, n, a->dw_max, a->dw, a->counts);
+      hipLaunchKernelGGL(hebbian_reduce_kernel, dim3(h.nK, (h.N + 255) / 256), dim3(256),
+            a->counts ? (size_t)a->nyp * a->nxp * sizeof(int) : 0, s, part, h.diff, pl.chunks, h.N, a->nyp, a->nxp,
+            a->nfp, a->dw_max, a->dw, a->counts);
       PVHIP_LAUNCHED("hebbian_reduce");
       return PVHIP_OK;
    }
@@ -577,7 +730,7 @@ size_t pvhip_hebbian_dw_scratch_bytes(const pvhip_hebbian_args *a) {
       return 0;
    }
    HebbPlan pl = hebb_plan(*a, a->arith == PVHIP_ARITH_BF16);
-   return pl.partBytes * (a->counts ? 2 : 1);
+   return pl.partBytes + pl.diffBytes;
 }
 
 } // extern "C"

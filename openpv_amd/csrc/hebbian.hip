@@ -104,32 +104,54 @@ __global__ void __launch_bounds__(256) hebbian_exact_kernel(HebbParams p) {
 // 8 x 128x128x1024 -> 16x16 in BF16, and 96 beside 65 us for
 // 7 x 45x37x200 -> 8x8x3 in FP32.)
 //
-// Workgroup: 64 features x 256 items, 4 waves; wave w owns items
-// 64w .. 64w+63 (4 MFMA column blocks) for all 64 features (4 row blocks).
-// K runs over pre extended rows (b, ye); per row the 64-feature activity
-// slab is staged transposed in LDS ([f][xe], T) and the post rows of the
-// windows are staged phase-split ([ky][f'][phase][xq], T) so that the values
-// for 8 consecutive pre columns xe of one item are 8 consecutive LDS
-// elements.  A lane's 8 K values are pre columns 8g..8g+7 of a 32-column
-// step; the FP32 form runs eight v_mfma_f32_16x16x4f32, MFMA j taking column
-// 8g+j (the same permutation of K for both operands).  BF16 rows are stored
-// twice, the second copy shifted by one element, so a fragment starting at
-// any element is read as four aligned 32-bit words.
+// Workgroup: 64 features x up to 256 items (NB blocks of 16), 4 waves; wave w
+// owns features 16w .. 16w+15 for all the items.  K runs over pre extended rows
+// (b, ye), 32 columns xe a step.  The A operand (activity) needs no LDS: lane
+// (r, g) loads the activity of feature r at columns 8g .. 8g+7, each load a run
+// of 16 features per column, HPF steps ahead, and converts it in registers.
+// The post rows of the windows are staged in LDS phase-split
+// ([ring row][f'][phase][xq], T) so that the values for 8 consecutive pre
+// columns xe of one item are 8 consecutive LDS elements; they live in a ring
+// (slot = post row mod R), so a pre row following the one before in the same
+// image stages only the sy post rows its window advanced by.  With R = nyp + sy
+// those are written while the current row is still being read: one barrier a
+// row (R = nyp, where the LDS has no room for more, needs two).  A thread's
+// elements of a post row are the same for every row, so their offsets are
+// computed once.  A lane's 8 K values are pre columns 8g..8g+7 of a step; the
+// FP32 form runs eight v_mfma_f32_16x16x4f32, MFMA j taking column 8g+j (the
+// same permutation of K for both operands).  BF16 rows are stored twice, the
+// second copy shifted by one element, so a fragment starting at any element is
+// read as four aligned 32-bit words.
+//
+// Bound: no single unit; with parts left out in turn, the LDS reads of the
+// window fragments, the staging between barriers and the MFMAs cost about a
+// fifth each of the large case.  Measured against the form that staged the
+// activity through LDS (two barriers and two thousand index instructions a
+// row): 8 x 128x128x1024 -> 16x16 BF16 409 -> 277 us, 7 x 45x37x200 -> 8x8x3
+// FP32 69 -> 49 us.
 constexpr int HMT = 64;  // features per workgroup
-constexpr int HNT = 256; // items per workgroup
-constexpr int HNB = HNT / 4 / 16; // 16-item blocks per wave
+constexpr int HNT = 256; // items per workgroup (at most)
+constexpr int HPF = 2;   // steps whose activity is in flight
+constexpr int HBR = 4;   // post rows and elements per thread prefetched for the next pre row
+constexpr int HBI = 3;
 
 struct HebbMfma {
    Geo pre, post;
    int nxp, nyp, nfp, N, nK;
    int sx, cx0, qx0, sy, cy; // window: post ext x = sx*(xq + qx0) + phase, rows sy*ye + cy + ky
-   int kxPad, lq, apitch;     // 32-padded pre ext width, B row length, A row pitch (elements)
+   int kxPad, lq, ring;       // 32-padded pre ext width, B row length, ring rows
    int rowsPerChunk;
    const float *preData, *postData;
    float *part; // [chunks][nK][N]
    int *diff;   // [nyp][nxp][nK] differences of the activation counts, or NULL
    int xA, xB, yA, yB; // pre extended columns and rows whose whole window is inside
+   float iNfp, iNxp, iSx; // reciprocals of nfp, nxp, sx
 };
+
+// n / d by the reciprocal of d, exact for 0 <= n < 2^21 (the items, columns and
+// LDS elements of a workgroup): three instructions where an integer division
+// by a runtime value takes about forty, and a workgroup's start needs many.
+__device__ __forceinline__ int hdiv(int n, float inv) { return (int)(((float)n + 0.5f) * inv); }
 
 template <typename T>
 struct HebbFrag;
@@ -142,52 +164,28 @@ struct HebbFrag<float> {
    typedef f32x8v type;
 };
 
-template <typename T>
-__device__ __forceinline__ T hcvt(float v) {
-   return (T)v;
-}
-
-// B fragment: 8 consecutive elements of a B row starting at element e.
-template <typename T>
-__device__ __forceinline__ typename HebbFrag<T>::type hload_b(const T *bl, int copyStride, int e);
-template <>
-__device__ __forceinline__ bf16x8v hload_b<__bf16>(const __bf16 *bl, int copyStride, int e) {
-   // copy 1 holds row[j + 1] at j: an odd start is an even start there
-   const __bf16 *p = (e & 1) ? bl + copyStride + e - 1 : bl + e;
+// B fragment: 8 consecutive elements at p (4-byte aligned).
+__device__ __forceinline__ bf16x8v hload_b(const __bf16 *p) {
    const uint32_t *w = reinterpret_cast<const uint32_t *>(p);
    uint32_t v[4] = {w[0], w[1], w[2], w[3]};
    return __builtin_bit_cast(bf16x8v, v);
 }
-template <>
-__device__ __forceinline__ f32x8v hload_b<float>(const float *bl, int, int e) {
+__device__ __forceinline__ f32x8v hload_b(const float *p) {
    f32x8v v;
 #pragma unroll
    for (int j = 0; j < 8; j++) {
-      v[j] = bl[e + j];
+      v[j] = p[j];
    }
    return v;
 }
 
-// Staging of a pre row, software-pipelined: the next row's activity values
-// and window values are loaded into registers (HAREG and HBR x HBX per
-// thread, any rest loaded when stored) while the MFMAs of the current row run.  The window's post rows sit in a
-// ring of nyp rows (slot = post row mod nyp), so a pre row following the one
-// before in the same image stages only the post rows the window advanced by
-// (sy of them), not all nyp.
-constexpr int HAREG = 32;
-// window values held per lane: HBR B rows per wave (B row = post row, feature,
-// phase) x HBX values 64 apart along the row
-constexpr int HBR = 4;
-constexpr int HBX = 3;
-
-template <typename T>
+template <typename T, int NB>
 __global__ void __launch_bounds__(256, 2) hebbian_mfma_kernel(HebbMfma h) {
    extern __shared__ float smem[];
-   int const copies = sizeof(T) == 2 ? 2 : 1;
-   int const nbrow  = h.nyp * h.nfp * h.sx; // B rows (ring slot, feature, phase)
-   int const cstr   = (nbrow * h.lq + 7) / 8 * 8; // elements per B copy (16-byte multiple)
+   using Frag       = typename HebbFrag<T>::type;
    T *bl            = reinterpret_cast<T *>(smem);
-   T *al            = bl + (size_t)copies * cstr; // [HMT][apitch]
+   int const rowB   = h.nfp * h.sx * h.lq;                // B elements of one post row
+   int const cstr   = (h.ring * rowB + 7) / 8 * 8;        // elements per B copy (16-byte multiple)
    int const f0     = blockIdx.x * HMT;
    int const n0     = blockIdx.y * HNT;
    int const chunk  = blockIdx.z;
@@ -198,239 +196,300 @@ __global__ void __launch_bounds__(256, 2) hebbian_mfma_kernel(HebbMfma h) {
    int const r1     = min(r0 + h.rowsPerChunk, rows);
    int const tid    = threadIdx.x;
    int const lane   = tid % 64;
-   int const wave   = tid / 64;
+   int const wave   = __builtin_amdgcn_readfirstlane(tid / 64);
    int const r      = lane % 16;
    int const g      = lane / 16;
    int const nxExtP = h.post.nxExt();
-   int const rowB   = h.nfp * h.sx * h.lq; // B elements of one post row
-   int const aItems = HMT * h.kxPad;
 
-   // this lane's item of each item block: window row ky, feature fp, and the
-   // B element offset within a ring slot
-   int nky[HNB], nsub[HNB];
+   // this lane's item of each item block: window row (upper bits) and the B
+   // element offset within a ring row (an odd one in the shifted copy)
+   constexpr int KYS = 20; // bits of an LDS element offset
+   int item[NB];
 #pragma unroll
-   for (int nb = 0; nb < HNB; nb++) {
-      int n     = min(n0 + (wave * HNB + nb) * 16 + r, h.N - 1);
-      int fp    = n % h.nfp;
-      int kx    = (n / h.nfp) % h.nxp;
-      nky[nb]   = n / (h.nfp * h.nxp);
-      int ph    = (h.cx0 + kx) % h.sx;
-      nsub[nb]  = (fp * h.sx + ph) * h.lq + (h.cx0 + kx) / h.sx + 8 * g;
+   for (int nb = 0; nb < NB; nb++) {
+      int const n  = min(n0 + nb * 16 + r, h.N - 1);
+      int const kp = hdiv(n, h.iNfp); // ky*nxp + kx
+      int const fp = n - kp * h.nfp;
+      int const ky = hdiv(kp, h.iNxp);
+      int const px = h.cx0 + kp - ky * h.nxp;
+      int const xq = hdiv(px, h.iSx);
+      int sub      = (fp * h.sx + px - xq * h.sx) * h.lq + xq + 8 * g;
+      if (sizeof(T) == 2 && (sub & 1)) { // lq and x0 are even: the parity stays
+         sub += cstr - 1;
+      }
+      item[nb] = ky << KYS | sub;
    }
-   f32x4 acc[4][HNB];
+   f32x4 acc[NB];
 #pragma unroll
-   for (int mb = 0; mb < 4; mb++) {
-#pragma unroll
-      for (int nb = 0; nb < HNB; nb++) {
-         acc[mb][nb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-      }
+   for (int nb = 0; nb < NB; nb++) {
+      acc[nb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
    }
-   auto ring = [&](int py) { int m = py % h.nyp; return m < 0 ? m + h.nyp : m; };
-   // activity element i (feature m = i % HMT, pre column xe = i / HMT) of pre row `row`
-   auto a_val = [&](int row, int i) -> float {
-      int const b  = row / nyExt;
-      int const ye = row % nyExt;
-      int const m  = i % HMT;
-      int const xe = i / HMT;
-      float v      = 0.0f;
-      if (xe < nxExt && f0 + m < h.nK) {
-         v = h.preData[(((size_t)b * nyExt + ye) * nxExt + xe) * h.pre.nf + f0 + m];
+
+   // ---- post rows -> LDS.  Element i of a post row is post column i / nfp of
+   // the staged range, feature i % nfp.
+   int const bItems = h.sx * h.lq * h.nfp;
+   auto b_item = [&](int i, int &loff, int &goff) {
+      int const pxr = hdiv(i, h.iNfp);
+      int const c   = i - pxr * h.nfp;
+      int const px  = pxr + h.sx * h.qx0;
+      int const xq  = hdiv(pxr, h.iSx);
+      loff          = (c * h.sx + pxr - xq * h.sx) * h.lq + xq;
+      goff          = px >= h.post.lt && px < h.post.lt + h.post.nx ? px * h.nfp + c : -1;
+   };
+   int bL[HBI], bG[HBI]; // offsets of this thread's first HBI elements
+#pragma unroll
+   for (int u = 0; u < HBI; u++) {
+      int const i = tid + 256 * u;
+      b_item(min(i, bItems - 1), bL[u], bG[u]);
+      bL[u] = i < bItems ? bL[u] : -1;
+   }
+   auto slot_of = [&](int py) {
+      int const m = py % h.ring;
+      return m < 0 ? m + h.ring : m;
+   };
+   auto wrap = [&](int slot) {
+      while (slot >= h.ring) {
+         slot -= h.ring;
       }
-      return v;
+      return slot;
    };
-   // post rows a pre row stages: [pyA, pyB) (all nyp rows, or the sy new ones
-   // when the row before was the previous pre row of the same image)
-   auto new_rows = [&](int row, int &pyA, int &pyB) {
-      int const ye = row % nyExt;
-      int const wy = h.sy * ye + h.cy;
-      pyA          = wy;
-      pyB          = wy + h.nyp;
-      if (row > r0 && ye > 0 && h.sy < h.nyp) {
-         pyA = wy + h.nyp - h.sy;
-      }
+   // post row py of batch element b, or NULL outside the restricted rows
+   auto post_row = [&](int b, int py) -> const float * {
+      return py >= h.post.up && py < h.post.up + h.post.ny
+                   ? h.postData + (size_t)b * h.post.numExt() + (size_t)py * nxExtP * h.nfp
+                   : nullptr;
    };
-   // element tid + 256*u of the activity slab is feature tid % HMT of pre
-   // column tid / HMT + 4*u (256 is a multiple of HMT)
-   static_assert(256 % HMT == 0, "activity slab walk assumes HMT divides 256");
-   int const am  = tid % HMT;
-   int const ax0 = tid / HMT;
-   // window value (B row br of the staged post rows [pyA, ..), position xq),
-   // and its ring slot; B rows are walked one per wave, lanes along xq, so the
-   // row's decomposition is wave-uniform
-   auto b_row = [&](int row, int pyA, int br, int &py, int &fp, int &ph) {
-      int const pr = h.nfp * h.sx;
-      py           = pyA + br / pr;
-      fp           = (br % pr) / h.sx;
-      ph           = br % h.sx;
-   };
-   auto b_elem = [&](int b, int py, int fp, int ph, int xq) -> float {
-      int const px = h.sx * (xq + h.qx0) + ph;
-      bool const in = py >= h.post.up && py < h.post.up + h.post.ny && px >= h.post.lt
-                      && px < h.post.lt + h.post.nx;
-      return in ? h.postData[(size_t)b * h.post.numExt() + ((size_t)py * nxExtP + px) * h.post.nf + fp] : 0.0f;
-   };
-   auto b_put = [&](int py, int fp, int ph, int xq, float v) {
-      int const idx = ring(py) * rowB + (fp * h.sx + ph) * h.lq + xq;
-      T const t     = hcvt<T>(v);
-      bl[idx]       = t;
-      if (copies == 2 && xq > 0) {
-         bl[cstr + idx - 1] = t; // copy 1: row shifted left by one element
+   auto b_get = [&](const float *P, int goff) { return P && goff >= 0 ? P[goff] : 0.0f; };
+   auto b_put = [&](int slot, int loff, float v) {
+      int const idx = slot * rowB + loff;
+      T const x     = (T)v;
+      bl[idx]       = x;
+      if (sizeof(T) == 2 && idx > 0) {
+         bl[cstr + idx - 1] = x; // copy 1: shifted left by one element
       }
    };
-   float va[HAREG], vb[HBR][HBX];
-   auto fetch = [&](int row) {
-      int pyA, pyB;
-      new_rows(row, pyA, pyB);
-      int const nbr = (pyB - pyA) * h.nfp * h.sx; // B rows to stage
-      int const b   = row / nyExt;
+   auto stage_rest = [&](const float *P, int slot) __attribute__((always_inline)) { // elements past the prefetched ones
+      for (int i = tid + 256 * HBI; i < bItems; i += 256) {
+         int lo, go;
+         b_item(i, lo, go);
+         b_put(slot, lo, b_get(P, go));
+      }
+   };
+   // n post rows from py: the first HBR of them into registers, then to LDS
+   float vb[HBR][HBI];
+   auto fetch_rows = [&](int b, int py, int n) __attribute__((always_inline)) {
 #pragma unroll
       for (int j = 0; j < HBR; j++) {
-         int const br = wave + 4 * j;
-         int py = 0, fp = 0, ph = 0;
-         b_row(row, pyA, min(br, max(nbr - 1, 0)), py, fp, ph);
+         const float *P = j < n ? post_row(b, py + j) : nullptr;
 #pragma unroll
-         for (int x = 0; x < HBX; x++) {
-            int const xq = lane + 64 * x;
-            vb[j][x]     = (br < nbr && xq < h.lq) ? b_elem(b, py, fp, ph, xq) : 0.0f;
+         for (int u = 0; u < HBI; u++) {
+            vb[j][u] = bL[u] >= 0 ? b_get(P, bG[u]) : 0.0f;
          }
-      }
-      float const *base = h.preData + ((size_t)row * nxExt + ax0) * h.pre.nf + f0 + am; // row = b*nyExt + ye
-      bool const fok    = f0 + am < h.nK;
-#pragma unroll
-      for (int u = 0; u < HAREG; u++) {
-         int const xe = ax0 + (256 / HMT) * u;
-         float v      = 0.0f;
-         if (fok && xe < nxExt) {
-            v = base[(size_t)(256 / HMT) * u * h.pre.nf];
-         }
-         va[u] = v;
       }
    };
-   bool const counting = h.diff != nullptr && blockIdx.y == 0;
-   int active          = 0; // active neurons of feature f0 + am with a whole window
-   auto stage = [&](int row) {
-      int const ye     = row % nyExt;
-      bool const whole = counting && ye >= h.yA && ye < h.yB;
+   // (slot: ring row of post row py)
+   auto put_rows = [&](int b, int py, int slot, int n) __attribute__((always_inline)) {
 #pragma unroll
-      for (int u = 0; u < HAREG; u++) {
-         int const i = tid + 256 * u;
-         if (i < aItems) {
-            al[(i % HMT) * h.apitch + i / HMT] = hcvt<T>(va[u]);
-         }
-      }
-      if (whole) {
+      for (int j = 0; j < HBR; j++) {
+         if (j < n) {
 #pragma unroll
-         for (int u = 0; u < HAREG; u++) { // pre column wave + 4*u, the same for the whole wave
-            int const xe = wave + (256 / HMT) * u;
-            if (xe >= h.xA && xe < h.xB) {
-               active += va[u] != 0.0f ? 1 : 0;
-            }
-         }
-      }
-      for (int i = tid + 256 * HAREG; i < aItems; i += 256) {
-         float const v = a_val(row, i);
-         al[(i % HMT) * h.apitch + i / HMT] = hcvt<T>(v);
-         if (whole && i / HMT >= h.xA && i / HMT < h.xB) {
-            active += v != 0.0f ? 1 : 0;
-         }
-      }
-      int pyA, pyB;
-      new_rows(row, pyA, pyB);
-      int const nbr = (pyB - pyA) * h.nfp * h.sx;
-      int const b   = row / nyExt;
-      for (int br = wave; br < nbr; br += 4) {
-         int py, fp, ph;
-         b_row(row, pyA, br, py, fp, ph);
-         int const j = br / 4; // register slot of this B row, if any
-         for (int xq = lane; xq < h.lq; xq += 64) {
-            int const x = xq / 64;
-            float v;
-            if (j < HBR && x < HBX) {
-               // the prefetched value (the register index is a compile-time
-               // choice: select among the slots)
-               v = 0.0f;
-#pragma unroll
-               for (int jj = 0; jj < HBR; jj++) {
-#pragma unroll
-                  for (int xx = 0; xx < HBX; xx++) {
-                     v = (jj == j && xx == x) ? vb[jj][xx] : v;
-                  }
+            for (int u = 0; u < HBI; u++) {
+               if (bL[u] >= 0) {
+                  b_put(slot, bL[u], vb[j][u]);
                }
             }
-            else {
-               v = b_elem(b, py, fp, ph, xq);
-            }
-            b_put(py, fp, ph, xq, v);
+            stage_rest(post_row(b, py + j), slot);
+            slot = slot + 1 < h.ring ? slot + 1 : 0;
          }
+      }
+   };
+   auto stage_rows = [&](int b, int py, int slot, int n) __attribute__((always_inline)) {
+      for (int j = 0; j < n; j += HBR) {
+         fetch_rows(b, py + j, n - j);
+         put_rows(b, py + j, wrap(slot + j), n - j);
+      }
+   };
+   // The current pre row: batch element, row, its window's first post row and
+   // that row's ring slot.  The next row of the image continues its window: sy
+   // new post rows.
+   int cb = r0 / nyExt, ye = r0 - cb * nyExt;
+   int wy = h.sy * ye + h.cy, slot0 = slot_of(wy);
+   auto continues = [&]() { return ye + 1 < nyExt && h.sy < h.nyp; };
+   auto fetch_new = [&]() __attribute__((always_inline)) { fetch_rows(cb, wy + h.nyp, h.sy); };
+   auto stage_new = [&]() __attribute__((always_inline)) { // before the step to that row
+      put_rows(cb, wy + h.nyp, wrap(slot0 + h.nyp), h.sy);
+      stage_rows(cb, wy + h.nyp + HBR, wrap(slot0 + h.nyp + HBR), h.sy - HBR);
+   };
+   auto stage_window = [&]() __attribute__((always_inline)) { stage_rows(cb, wy, slot0, h.nyp); };
+   auto next_row = [&]() {
+      if (++ye < nyExt) {
+         wy += h.sy;
+         slot0 = wrap(slot0 + h.sy);
+      }
+      else {
+         ye = 0;
+         cb++;
+         wy    = h.cy;
+         slot0 = slot_of(wy);
+      }
+   };
+
+   // ---- activity: step q of the chunk is row r0 + q / steps, columns
+   // 32*(q % steps) ..; the loads of step q + HPF are issued in step q
+   int const steps  = h.kxPad / 32;
+   int const nSteps = (r1 - r0) * steps;
+   int const f      = min(f0 + wave * 16 + r, h.nK - 1); // rows past the last feature are not stored
+   float va[HPF][8];
+   int lRow = r0, lX = 0; // of the next load
+   uint32_t aoff[8];      // element of column 8g + j of a step
+#pragma unroll
+   for (int j = 0; j < 8; j++) {
+      aoff[j] = (uint32_t)((8 * g + j) * h.nK + f);
+   }
+   auto load_a = [&](float (&v)[8]) __attribute__((always_inline)) {
+      float const *base = h.preData + ((size_t)lRow * nxExt + lX) * h.nK;
+      if (lX + 32 <= nxExt) {
+#pragma unroll
+         for (int j = 0; j < 8; j++) {
+            v[j] = base[aoff[j]];
+         }
+      }
+      else { // columns past the layer read its last one and are cleared before use
+#pragma unroll
+         for (int j = 0; j < 8; j++) {
+            v[j] = base[(uint32_t)(min(8 * g + j, nxExt - 1 - lX) * h.nK + f)];
+         }
+      }
+      lX += 32;
+      if (lX >= h.kxPad) {
+         lX   = 0;
+         lRow = min(lRow + 1, r1 - 1); // past the end: loaded, not used
+      }
+   };
+   bool const counting = h.diff != nullptr && blockIdx.y == 0 && f0 + wave * 16 + r < h.nK;
+   int active          = 0; // active neurons of feature f with a whole window
+   if (r0 < r1) {
+#pragma unroll
+      for (int s = 0; s < HPF; s++) {
+         load_a(va[s]);
+      }
+      stage_window();
+   }
+   __syncthreads();
+   int row = r0, x0 = 0;
+   int bb[NB]; // B element of this row's fragments at column 0
+   auto bases = [&]() __attribute__((always_inline)) {
+#pragma unroll
+      for (int nb = 0; nb < NB; nb++) {
+         int s  = slot0 + (item[nb] >> KYS);
+         s      = s >= h.ring ? s - h.ring : s;
+         bb[nb] = s * rowB + (item[nb] & ((1 << KYS) - 1));
       }
    };
    if (r0 < r1) {
-      fetch(r0);
+      bases();
    }
-   for (int row = r0; row < r1; row++) {
-      __syncthreads(); // the previous row's fragments are consumed
-      stage(row);
-      __syncthreads();
-      if (row + 1 < r1) {
-         fetch(row + 1); // in flight during this row's MFMAs
-      }
-      int const wy = h.sy * (row % nyExt) + h.cy;
-      int bbase[HNB];
+   for (int q0 = 0; q0 < nSteps; q0 += HPF) {
 #pragma unroll
-      for (int nb = 0; nb < HNB; nb++) {
-         bbase[nb] = ring(wy + nky[nb]) * rowB + nsub[nb];
-      }
-      for (int x0 = 0; x0 < h.kxPad; x0 += 32) {
-         typename HebbFrag<T>::type af[4], bf[HNB];
-#pragma unroll
-         for (int mb = 0; mb < 4; mb++) {
-            T const *ap = al + (mb * 16 + r) * h.apitch + x0 + 8 * g;
-            if constexpr (sizeof(T) == 2) {
-               af[mb] = *reinterpret_cast<const bf16x8v *>(ap);
+      for (int s = 0; s < HPF; s++) {
+         if (q0 + s < nSteps) { // the same for the whole workgroup
+            if (x0 == 0 && row + 1 < r1 && continues()) {
+               fetch_new(); // in flight during this row
             }
-            else {
-               f32x4 lo = *reinterpret_cast<const f32x4 *>(ap);
-               f32x4 hi = *reinterpret_cast<const f32x4 *>(ap + 4);
-               af[mb]   = f32x8v{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+            bool const tail = x0 + 32 > nxExt;
+            if (tail) { // columns past the layer
+#pragma unroll
+               for (int j = 0; j < 8; j++) {
+                  va[s][j] = x0 + 8 * g + j < nxExt ? va[s][j] : 0.0f;
+               }
             }
-         }
+            if (counting && ye >= h.yA && ye < h.yB) {
+               if (x0 >= h.xA && x0 + 32 <= h.xB) {
 #pragma unroll
-         for (int nb = 0; nb < HNB; nb++) {
-            bf[nb] = hload_b<T>(bl, cstr, bbase[nb] + x0);
-         }
-#pragma unroll
-         for (int mb = 0; mb < 4; mb++) {
-#pragma unroll
-            for (int nb = 0; nb < HNB; nb++) {
-               if constexpr (sizeof(T) == 2) {
-                  acc[mb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[mb], bf[nb], acc[mb][nb], 0, 0, 0);
+                  for (int j = 0; j < 8; j++) {
+                     active += va[s][j] != 0.0f ? 1 : 0;
+                  }
                }
                else {
 #pragma unroll
                   for (int j = 0; j < 8; j++) {
-                     acc[mb][nb] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[mb][j], bf[nb][j], acc[mb][nb], 0, 0, 0);
+                     int const xe = x0 + 8 * g + j;
+                     active += va[s][j] != 0.0f && xe >= h.xA && xe < h.xB ? 1 : 0;
                   }
+               }
+            }
+            Frag af;
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+               af[j] = (T)va[s][j];
+            }
+            load_a(va[s]); // step q0 + s + HPF
+            // B fragments a group ahead of their MFMAs
+            constexpr int G = sizeof(T) == 2 ? 4 : 1;
+            Frag bf[2][G];
+#pragma unroll
+            for (int k = 0; k < G; k++) {
+               bf[0][k] = hload_b(bl + bb[k] + x0);
+            }
+#pragma unroll
+            for (int nb = 0; nb < NB; nb += G) {
+#pragma unroll
+               for (int k = 0; k < G; k++) {
+                  if (nb + G < NB) {
+                     bf[(nb / G + 1) % 2][k] = hload_b(bl + bb[(nb + G) % NB + k] + x0);
+                  }
+               }
+               __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+               for (int k = 0; k < G; k++) {
+                  Frag const b = bf[nb / G % 2][k];
+                  if constexpr (sizeof(T) == 2) {
+                     acc[nb + k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, b, acc[nb + k], 0, 0, 0);
+                  }
+                  else {
+#pragma unroll
+                     for (int j = 0; j < 8; j++) {
+                        acc[nb] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[j], b[j], acc[nb], 0, 0, 0);
+                     }
+                  }
+               }
+            }
+            x0 += 32;
+            if (x0 >= h.kxPad) { // the next row
+               x0 = 0;
+               if (row + 1 < r1) {
+                  bool const next = continues();
+                  if (!next || h.ring == h.nyp) {
+                     __syncthreads(); // this row's fragments are consumed
+                  }
+                  row++;
+                  if (next) {
+                     stage_new();
+                  }
+                  next_row();
+                  if (!next) {
+                     stage_window();
+                  }
+                  __syncthreads();
+                  bases();
                }
             }
          }
       }
    }
-   if (active > 0) { // va is 0 past the last feature
-      atomicAdd(h.diff + f0 + am, active);
+   if (counting && active > 0) {
+      atomicAdd(h.diff + f, active);
    }
-   // D[4g+i][r]: feature f0 + mb*16 + 4g + i, item of lane r in block nb
+   // D[4g+i][r]: feature f0 + 16*wave + 4g + i, item of lane r in block nb
    float *out = h.part + (size_t)chunk * h.nK * h.N;
 #pragma unroll
-   for (int mb = 0; mb < 4; mb++) {
+   for (int nb = 0; nb < NB; nb++) {
+      int const n = n0 + nb * 16 + r;
 #pragma unroll
-      for (int nb = 0; nb < HNB; nb++) {
-         int const n = n0 + (wave * HNB + nb) * 16 + r;
-#pragma unroll
-         for (int i = 0; i < 4; i++) {
-            int const f = f0 + mb * 16 + 4 * g + i;
-            if (f < h.nK && n < h.N) {
-               out[(size_t)f * h.N + n] = acc[mb][nb][i];
-            }
+      for (int i = 0; i < 4; i++) {
+         int const fo = f0 + wave * 16 + 4 * g + i;
+         if (fo < h.nK && n < h.N) {
+            out[(size_t)fo * h.N + n] = acc[nb][i];
          }
       }
    }
@@ -566,7 +625,7 @@ __global__ void __launch_bounds__(256) hebbian_reduce_kernel(
 }
 
 struct HebbPlan {
-   int chunks, rowsPerChunk, kxPad, lq, apitch;
+   int chunks, rowsPerChunk, kxPad, lq, ring;
    size_t lds, partBytes;
    size_t diffBytes; // difference array of the counts
 };
@@ -591,11 +650,18 @@ HebbPlan hebb_plan(const pvhip_hebbian_args &a, bool bf) {
    int qx0         = cx >= 0 ? cx / sx : -((-cx + sx - 1) / sx);
    int cx0         = cx - sx * qx0;
    pl.lq           = (pl.kxPad + (cx0 + a.nxp - 1) / sx + 2 + 1) / 2 * 2;
-   pl.apitch       = pl.kxPad + 8;
    size_t esz      = bf ? 2 : 4;
    int copies      = bf ? 2 : 1;
-   size_t cstr     = ((size_t)a.nyp * a.nfp * sx * pl.lq + 7) / 8 * 8;
-   pl.lds          = ((size_t)copies * cstr + (size_t)HMT * pl.apitch) * esz;
+   auto lds_of     = [&](int ring) {
+      return copies * (((size_t)ring * a.nfp * sx * pl.lq + 7) / 8 * 8) * esz;
+   };
+   // room for the rows of the next window beside the current one's, unless
+   // that leaves one workgroup per CU
+   pl.ring = a.nyp + std::max(1, a.window_stride_y);
+   if (lds_of(pl.ring) > 80 * 1024) {
+      pl.ring = a.nyp;
+   }
+   pl.lds = lds_of(pl.ring);
    pl.partBytes    = (size_t)pl.chunks * nK * N * sizeof(float);
    pl.diffBytes    = a.counts ? (size_t)nK * a.nyp * a.nxp * sizeof(int) : 0;
    return pl;
@@ -646,7 +712,10 @@ int pvhip_hebbian_dw(const pvhip_hebbian_args *a, pvhip_stream stream) {
       h.cy      = a->window_start_y;
       h.kxPad   = pl.kxPad;
       h.lq      = pl.lq;
-      h.apitch  = pl.apitch;
+      h.ring    = pl.ring;
+      h.iNfp    = 1.0f / (float)h.nfp;
+      h.iNxp    = 1.0f / (float)h.nxp;
+      h.iSx     = 1.0f / (float)h.sx;
       h.rowsPerChunk = pl.rowsPerChunk;
       h.preData  = a->pre_data;
       h.postData = a->post_data;
@@ -672,12 +741,22 @@ int pvhip_hebbian_dw(const pvhip_hebbian_args *a, pvhip_stream stream) {
          whole(a->window_start_x, h.sx, h.post.lt, h.post.nx, h.nxp, h.pre.nxExt(), h.xA, h.xB);
          whole(a->window_start_y, h.sy, h.post.up, h.post.ny, h.nyp, h.pre.nyExt(), h.yA, h.yB);
       }
-      if (bf) {
-         hipLaunchKernelGGL(hebbian_mfma_kernel<__bf16>, grid, dim3(256), pl.lds, s, h);
-      }
-      else {
-         hipLaunchKernelGGL(hebbian_mfma_kernel<float>, grid, dim3(256), pl.lds, s, h);
-      }
+      // item blocks of 16 a workgroup holds accumulators for
+      int const nb = (std::min(h.N, HNT) + 15) / 16;
+#define PVHIP_HEBB(NBV)                                                                                  \
+   do {                                                                                                 \
+      if (bf) {                                                                                         \
+         hipLaunchKernelGGL((hebbian_mfma_kernel<__bf16, NBV>), grid, dim3(256), pl.lds, s, h);          \
+      }                                                                                                 \
+      else {                                                                                            \
+         hipLaunchKernelGGL((hebbian_mfma_kernel<float, NBV>), grid, dim3(256), pl.lds, s, h);           \
+      }                                                                                                 \
+   } while (0)
+      if (nb <= 4) PVHIP_HEBB(4);
+      else if (nb <= 8) PVHIP_HEBB(8);
+      else if (nb <= 12) PVHIP_HEBB(12);
+      else PVHIP_HEBB(16);
+#undef PVHIP_HEBB
       PVHIP_LAUNCHED("hebbian_mfma");
       if (h.diff) {
          long long const nbx = h.pre.nxExt() - (h.xB - h.xA), nby = h.pre.nyExt() - (h.yB - h.yA);

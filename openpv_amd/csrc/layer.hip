@@ -164,6 +164,140 @@ __global__ void __launch_bounds__(kRowThreads) ista_update_kernel(LCAParams p, f
    }
 }
 
+// The three LCA-layer updates above with 16-byte accesses: a thread takes four
+// consecutive neurons of a row (two such quads 256 threads apart, their loads
+// issued together), one division per quad for its row and one for its position
+// in the chunked BF16 copy.  Per neuron the operations are those of
+// lca_update_kernel, momentum_lca_update_kernel and ista_update_kernel, in
+// their order.  HBM-bound; 64 x 32x32x512, momentum rule (24 bytes per
+// neuron): 240 us (3.3 TB/s) with 4-byte accesses and two divisions per
+// neuron, 152 us here.
+enum : int { RULE_LCA = 0, RULE_MOMENTUM = 1, RULE_ISTA = 2 };
+constexpr int kQuads = 2;
+
+__device__ __forceinline__ void load4(const float *p, float (&v)[4]) {
+   float4 const x = *reinterpret_cast<const float4 *>(p);
+   v[0]           = x.x;
+   v[1]           = x.y;
+   v[2]           = x.z;
+   v[3]           = x.w;
+}
+__device__ __forceinline__ void store4(float *p, const float (&v)[4]) {
+   *reinterpret_cast<float4 *>(p) = make_float4(v[0], v[1], v[2], v[3]);
+}
+
+template <int RULE>
+__global__ void __launch_bounds__(kRowThreads)
+      lca_update_vec_kernel(LCAParams p, float param, float *prevDrive) {
+   int const numRes = p.loc.numRes();
+   int const rowLen = p.loc.nx * p.loc.nf;
+   int const b      = blockIdx.y;
+   size_t const n   = (size_t)p.loc.nbatch * numRes;
+   float const e    = p.expTau[b]; // ISTA: the rate
+   float V[kQuads][4], A[kQuads][4], D[kQuads][4], G[kQuads][PVHIP_MAX_CHANNELS][4];
+   size_t ai[kQuads];
+   int k[kQuads], y[kQuads];
+#pragma unroll
+   for (int u = 0; u < kQuads; u++) {
+      int const want  = ((blockIdx.x * kQuads + u) * kRowThreads + threadIdx.x) * 4;
+      k[u]            = min(want, numRes - 4); // past the end: loaded, not stored
+      y[u]            = k[u] / rowLen;
+      ai[u]           = ext_row(p.loc, b, y[u]) + (k[u] - y[u] * rowLen);
+      size_t const vi = (size_t)b * numRes + k[u];
+#pragma unroll
+      for (int ch = 0; ch < PVHIP_MAX_CHANNELS; ch++) {
+         if (ch < p.numChannels) {
+            load4(p.gsyn + (size_t)ch * n + vi, G[u][ch]);
+         }
+      }
+      load4(p.V + vi, V[u]);
+      if (!p.aFromV) {
+         load4(p.A + ai[u], A[u]);
+      }
+      if (RULE == RULE_MOMENTUM) {
+         load4(prevDrive + vi, D[u]);
+      }
+      k[u] = want;
+   }
+#pragma unroll
+   for (int u = 0; u < kQuads; u++) {
+      if (k[u] >= numRes) {
+         continue;
+      }
+      float vn[4], an[4], dn[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+         float g = 0.0f; // GSynAccumulator
+#pragma unroll
+         for (int ch = 0; ch < PVHIP_MAX_CHANNELS; ch++) {
+            if (ch < p.numChannels) {
+               float const prod = p.coeffs[ch] * G[u][ch][i];
+               g                = g + prod;
+            }
+         }
+         float const vo = V[u][i];
+         float const ao = p.aFromV ? apply_transfer(p.transfer, vo) : A[u][i];
+         if (RULE == RULE_ISTA) {
+            float sign = 0.0f;
+            if (ao != 0.0f) {
+               sign = ao / fabsf(ao);
+            }
+            float const thr   = param * sign;
+            float const drive = g - thr;
+            float const step  = e * drive;
+            vn[i]             = vo + step;
+         }
+         else {
+            float const t1    = e * vo;
+            float const t2    = 1.0f - e;
+            float const si    = p.selfInteract * ao;
+            float const t3    = g + si;
+            float const drive = t2 * t3;
+            float v           = t1 + drive;
+            if (RULE == RULE_MOMENTUM) {
+               float const mom = param * D[u][i];
+               v               = v + mom;
+               dn[i]           = drive;
+            }
+            vn[i] = v;
+         }
+         an[i] = apply_transfer(p.transfer, vn[i]);
+      }
+      size_t const vi = (size_t)b * numRes + k[u];
+      store4(p.V + vi, vn);
+      if (RULE == RULE_MOMENTUM) {
+         store4(prevDrive + vi, dn);
+      }
+      if (p.A) {
+         store4(p.A + ai[u], an);
+      }
+      if (p.Ab) { // four features of one 32-feature chunk
+         typedef __bf16 bf16x4v __attribute__((ext_vector_type(4)));
+         *reinterpret_cast<bf16x4v *>(p.Ab + bf16c_index(p.loc, b, (int)(ai[u] - (size_t)b * p.loc.numExt()))) =
+               bf16x4v{(__bf16)an[0], (__bf16)an[1], (__bf16)an[2], (__bf16)an[3]};
+      }
+   }
+}
+
+// Rows of a layer's extended buffer at p start on multiples of m values.
+inline bool rows_aligned(const Geo &x, const void *p, int m) {
+   return ((uintptr_t)p % (4 * m)) == 0 && (x.numExt() % m) == 0 && ((x.nxExt() * x.nf) % m) == 0
+          && (((x.up * x.nxExt() + x.lt) * x.nf) % m) == 0;
+}
+
+// The 16-byte form applies: whole quads in every row, buffers and rows on
+// 16-byte boundaries.  (Ab needs nf % 32 == 0 and 16-byte alignment already.)
+inline bool lca_vec_ok(const LCAParams &p, const float *prevDrive) {
+   return (p.loc.nx * p.loc.nf) % 4 == 0 && (uintptr_t)p.V % 16 == 0
+          && (p.numChannels == 0 || (uintptr_t)p.gsyn % 16 == 0) && (uintptr_t)prevDrive % 16 == 0
+          && (p.A == nullptr || rows_aligned(p.loc, p.A, 4));
+}
+
+inline dim3 quad_grid(const Geo &g) {
+   int const per = kRowThreads * kQuads * 4;
+   return dim3((unsigned)((g.numRes() + per - 1) / per), (unsigned)g.nbatch);
+}
+
 struct LayerParams {
    Geo loc;
    int numChannels;
@@ -210,6 +344,32 @@ __global__ void __launch_bounds__(kRowThreads)
       if (k < numRes) {
          int const y = k / rowLen;
          A[ext_row(loc, b, y) + (k - y * rowLen)] = apply_transfer(t, V[(size_t)b * numRes + k]);
+      }
+   }
+}
+
+// ann_activity_kernel with 16-byte accesses (as lca_update_vec_kernel).
+__global__ void __launch_bounds__(kRowThreads)
+      ann_activity_vec_kernel(Geo loc, Transfer t, const float *V, float *A) {
+   int const numRes = loc.numRes();
+   int const rowLen = loc.nx * loc.nf;
+   int const b      = blockIdx.y;
+   float v[kQuads][4];
+   int k[kQuads];
+#pragma unroll
+   for (int u = 0; u < kQuads; u++) {
+      k[u] = ((blockIdx.x * kQuads + u) * kRowThreads + threadIdx.x) * 4;
+      load4(V + (size_t)b * numRes + min(k[u], numRes - 4), v[u]);
+   }
+#pragma unroll
+   for (int u = 0; u < kQuads; u++) {
+      if (k[u] < numRes) {
+         int const y = k[u] / rowLen;
+#pragma unroll
+         for (int i = 0; i < 4; i++) {
+            v[u][i] = apply_transfer(t, v[u][i]);
+         }
+         store4(A + ext_row(loc, b, y) + (k[u] - y * rowLen), v[u]);
       }
    }
 }
@@ -901,7 +1061,13 @@ int pvhip_lca_update(const pvhip_lca_update_args *args, pvhip_stream stream) {
       return st;
    }
    PVHIP_REQUIRE(row_grid_ok(p.loc), "lca_update: more than 65535 rows or batch elements");
-   hipLaunchKernelGGL(lca_update_kernel, row_grid(p.loc), dim3(kRowThreads), 0, (hipStream_t)stream, p);
+   if (lca_vec_ok(p, nullptr)) {
+      hipLaunchKernelGGL(lca_update_vec_kernel<RULE_LCA>, quad_grid(p.loc), dim3(kRowThreads), 0,
+            (hipStream_t)stream, p, 0.0f, nullptr);
+   }
+   else {
+      hipLaunchKernelGGL(lca_update_kernel, row_grid(p.loc), dim3(kRowThreads), 0, (hipStream_t)stream, p);
+   }
    PVHIP_LAUNCHED("lca_update");
    return PVHIP_OK;
 }
@@ -917,8 +1083,14 @@ int pvhip_momentum_lca_update(
       return st;
    }
    PVHIP_REQUIRE(row_grid_ok(p.loc), "momentum_lca_update: more than 65535 batch elements");
-   hipLaunchKernelGGL(momentum_lca_update_kernel, row_grid(p.loc), dim3(kRowThreads), 0,
-         (hipStream_t)stream, p, momentum_rate, prev_drive);
+   if (lca_vec_ok(p, prev_drive)) {
+      hipLaunchKernelGGL(lca_update_vec_kernel<RULE_MOMENTUM>, quad_grid(p.loc), dim3(kRowThreads), 0,
+            (hipStream_t)stream, p, momentum_rate, prev_drive);
+   }
+   else {
+      hipLaunchKernelGGL(momentum_lca_update_kernel, row_grid(p.loc), dim3(kRowThreads), 0,
+            (hipStream_t)stream, p, momentum_rate, prev_drive);
+   }
    PVHIP_LAUNCHED("momentum_lca_update");
    return PVHIP_OK;
 }
@@ -931,8 +1103,14 @@ int pvhip_ista_update(const pvhip_lca_update_args *args, float vthresh, pvhip_st
       return st;
    }
    PVHIP_REQUIRE(row_grid_ok(p.loc), "ista_update: nbatch too large");
-   hipLaunchKernelGGL(ista_update_kernel, row_grid(p.loc), dim3(kRowThreads), 0, (hipStream_t)stream, p,
-         vthresh);
+   if (lca_vec_ok(p, nullptr)) {
+      hipLaunchKernelGGL(lca_update_vec_kernel<RULE_ISTA>, quad_grid(p.loc), dim3(kRowThreads), 0,
+            (hipStream_t)stream, p, vthresh, nullptr);
+   }
+   else {
+      hipLaunchKernelGGL(ista_update_kernel, row_grid(p.loc), dim3(kRowThreads), 0, (hipStream_t)stream, p,
+            vthresh);
+   }
    PVHIP_LAUNCHED("ista_update");
    return PVHIP_OK;
 }
@@ -1016,7 +1194,13 @@ int pvhip_ann_activity(
    }
    Geo g = geo(*loc);
    PVHIP_REQUIRE(row_grid_ok(g), "ann_activity: more than 65535 rows or batch elements");
-   hipLaunchKernelGGL(ann_activity_kernel, row_grid(g), dim3(kRowThreads), 0, (hipStream_t)stream, g, t, V, A);
+   if ((g.nx * g.nf) % 4 == 0 && (uintptr_t)V % 16 == 0 && rows_aligned(g, A, 4)) {
+      hipLaunchKernelGGL(ann_activity_vec_kernel, quad_grid(g), dim3(kRowThreads), 0, (hipStream_t)stream, g, t,
+            V, A);
+   }
+   else {
+      hipLaunchKernelGGL(ann_activity_kernel, row_grid(g), dim3(kRowThreads), 0, (hipStream_t)stream, g, t, V, A);
+   }
    PVHIP_LAUNCHED("ann_activity");
    return PVHIP_OK;
 }
@@ -1038,10 +1222,6 @@ int pvhip_error_update(const pvhip_error_update_args *a, pvhip_stream stream) {
    // 16-byte form when every row segment of four values is aligned for it:
    // rows of a multiple of 4 values, the inputs' and V's rows on 16-byte
    // boundaries, A's rows on multiples of 4 (else 2) values
-   auto rows_aligned = [](const Geo &x, const void *p, int m) {
-      return ((uintptr_t)p % (4 * m)) == 0 && (x.numExt() % m) == 0 && ((x.nxExt() * x.nf) % m) == 0
-             && (((x.up * x.nxExt() + x.lt) * x.nf) % m) == 0;
-   };
    Geo const gi = geo(a->in_loc), gr = geo(a->rec_loc);
    bool const vec = (g.nx * g.nf) % 4 == 0 && rows_aligned(gi, a->in, 4) && rows_aligned(gr, a->rec, 4)
                     && (uintptr_t)a->V % 16 == 0 && rows_aligned(g, a->A, 2);

@@ -501,11 +501,24 @@ __global__ void __launch_bounds__(kRowThreads) error_update_vec_kernel(
 // (DataStore.cpp:55-62).  Chunks of kChunk consecutive elements per
 // workgroup; pass 1 counts, pass 2 scans the chunk counts of each batch
 // element, pass 3 writes entries and the per-position segment starts.
+//
+// A chunk is ITERS rounds of the workgroup, with two barriers each in pass 3.
+// A small layer takes one round per chunk, so that it fills the chip instead
+// of a few workgroups walking 16 rounds; beyond kSmallChunks such chunks the
+// 16-round ones fill it too, with a sixteenth of the counts to scan (and the
+// counts of pvhip_active_compact_noalloc's fixed workspace go as far as they
+// did).  One image of 256x256x16: the list and its sparse delivery 66.4 us with
+// 16 rounds, 47.1 us with one.
 
 constexpr int kCompactThreads = 256;
 constexpr int kCompactIters   = 16;
 constexpr int kCompactVec     = 4; // elements per thread per iteration
-constexpr int kChunk          = kCompactThreads * kCompactIters * kCompactVec;
+constexpr int kSmallChunks    = 8192;
+
+inline int compact_iters(const Geo &g) {
+   int const one = kCompactThreads * kCompactVec;
+   return (long long)g.nbatch * ((g.numExt() + one - 1) / one) <= kSmallChunks ? 1 : kCompactIters;
+}
 
 // Loads elements [e, e+VEC) of one batch element's extended buffer (zeros past
 // the end); VEC == 4 requires numExt % 4 == 0 (16-byte aligned rows).
@@ -526,16 +539,17 @@ __device__ __forceinline__ void load_vec(const float *Ab, int e, int numExt, flo
    }
 }
 
-template <int VEC>
+template <int VEC, int ITERS>
 __global__ void __launch_bounds__(kCompactThreads)
       compact_count_kernel(const float *A, int numExt, uint32_t *chunkCount, int chunksPerBatch) {
+   constexpr int kChunk = kCompactThreads * ITERS * kCompactVec;
    int const b         = blockIdx.y;
    int const chunk     = blockIdx.x;
    float const *Ab     = A + (size_t)b * numExt;
    int const base      = chunk * kChunk;
    int count           = 0;
 #pragma unroll 4
-   for (int it = 0; it < kCompactIters; it++) {
+   for (int it = 0; it < ITERS; it++) {
       int e = base + (it * kCompactThreads + threadIdx.x) * kCompactVec;
       float a[kCompactVec];
       load_vec<VEC>(Ab, e, numExt, a);
@@ -568,7 +582,7 @@ __global__ void __launch_bounds__(1024)
       compact_scan_kernel(uint32_t *chunkCount, int chunksPerBatch, int64_t *numActive) {
    int const b        = blockIdx.x;
    uint32_t *c        = chunkCount + (size_t)b * chunksPerBatch;
-   __shared__ uint32_t partial[1024];
+   __shared__ uint32_t partial[1024 / kWave];
    int const per      = (chunksPerBatch + blockDim.x - 1) / blockDim.x;
    int const begin    = threadIdx.x * per;
    int const end      = min(begin + per, chunksPerBatch);
@@ -576,30 +590,38 @@ __global__ void __launch_bounds__(1024)
    for (int i = begin; i < end; i++) {
       local += c[i];
    }
-   partial[threadIdx.x] = local;
-   __syncthreads();
-   // Hillis-Steele inclusive scan over the per-thread sums.
-   for (int off = 1; off < (int)blockDim.x; off <<= 1) {
-      uint32_t v = threadIdx.x >= (unsigned)off ? partial[threadIdx.x - off] : 0u;
-      __syncthreads();
-      partial[threadIdx.x] += v;
-      __syncthreads();
+   // inclusive scan of the per-thread sums: within each wave, then over the waves
+   int const lane = threadIdx.x % kWave;
+   int const wave = threadIdx.x / kWave;
+   uint32_t incl  = local;
+#pragma unroll
+   for (int off = 1; off < kWave; off <<= 1) {
+      uint32_t const v = __shfl_up(incl, off, kWave);
+      incl += lane >= off ? v : 0u;
    }
-   uint32_t run = threadIdx.x > 0 ? partial[threadIdx.x - 1] : 0u;
+   if (lane == kWave - 1) {
+      partial[wave] = incl;
+   }
+   __syncthreads();
+   for (int w = 0; w < wave; w++) {
+      incl += partial[w];
+   }
+   uint32_t run = incl - local;
    for (int i = begin; i < end; i++) {
       uint32_t v = c[i];
       c[i]       = run;
       run += v;
    }
    if (threadIdx.x == blockDim.x - 1) {
-      numActive[b] = (int64_t)partial[blockDim.x - 1];
+      numActive[b] = (int64_t)incl;
    }
 }
 
-template <int VEC>
+template <int VEC, int ITERS>
 __global__ void __launch_bounds__(kCompactThreads) compact_write_kernel(
       const float *A, int numExt, int nf, const uint32_t *chunkOffset, int chunksPerBatch,
       pvhip_sparse_entry *entries, uint32_t *posStart, int numPos, const int64_t *numActive) {
+   constexpr int kChunk = kCompactThreads * ITERS * kCompactVec;
    int const b      = blockIdx.y;
    int const chunk  = blockIdx.x;
    float const *Ab  = A + (size_t)b * numExt;
@@ -610,7 +632,7 @@ __global__ void __launch_bounds__(kCompactThreads) compact_write_kernel(
    int const lane   = threadIdx.x % kWave;
    int const wave   = threadIdx.x / kWave;
    __shared__ uint32_t waveCount[kCompactThreads / kWave];
-   for (int it = 0; it < kCompactIters; it++) {
+   for (int it = 0; it < ITERS; it++) {
       int e = base + (it * kCompactThreads + threadIdx.x) * kCompactVec;
       float a[kCompactVec];
       load_vec<VEC>(Ab, e, numExt, a);
@@ -985,7 +1007,8 @@ __global__ void __launch_bounds__(256) activity_to_bf16c_kernel(Geo g, const flo
 } // namespace
 
 size_t compact_scratch_bytes(const Geo &g) {
-   return (size_t)g.nbatch * (size_t)((g.numExt() + kChunk - 1) / kChunk) * sizeof(uint32_t);
+   int const chunk = kCompactThreads * kCompactVec * compact_iters(g);
+   return (size_t)g.nbatch * (size_t)((g.numExt() + chunk - 1) / chunk) * sizeof(uint32_t);
 }
 
 int active_from_segments(
@@ -1296,33 +1319,37 @@ int compact_launch(const pvhip_loc &l, const float *A, pvhip_sparse_entry *entri
    const pvhip_loc *loc = &l;
    Geo g              = geo(*loc);
    int const numExt   = g.numExt();
-   int const chunks   = (numExt + kChunk - 1) / kChunk;
+   int const iters    = compact_iters(g);
+   int const chunk    = kCompactThreads * kCompactVec * iters;
+   int const chunks   = (numExt + chunk - 1) / chunk;
    int const numPos   = g.nxExt() * g.nyExt();
    PVHIP_REQUIRE(g.nbatch <= 65535, "active_compact: nbatch %d too large", g.nbatch);
    PVHIP_REQUIRE(chunk_scratch != nullptr, "active_compact: NULL chunk_scratch");
    uint32_t *scratch = chunk_scratch;
    dim3 grid(chunks, g.nbatch);
    bool const vec4 = numExt % 4 == 0 && ((uintptr_t)A & 15) == 0;
-   if (vec4) {
-      hipLaunchKernelGGL(compact_count_kernel<4>, grid, dim3(kCompactThreads), 0, (hipStream_t)stream,
-            A, numExt, scratch, chunks);
-   }
-   else {
-      hipLaunchKernelGGL(compact_count_kernel<1>, grid, dim3(kCompactThreads), 0, (hipStream_t)stream,
-            A, numExt, scratch, chunks);
-   }
+#define PVHIP_COUNT(V, I)                                                                                \
+   hipLaunchKernelGGL((compact_count_kernel<V, I>), grid, dim3(kCompactThreads), 0, (hipStream_t)stream, A, \
+         numExt, scratch, chunks)
+#define PVHIP_WRITE(V, I)                                                                                \
+   hipLaunchKernelGGL((compact_write_kernel<V, I>), grid, dim3(kCompactThreads), 0, (hipStream_t)stream, A, \
+         numExt, g.nf, scratch, chunks, entries, pos_start, numPos, num_active)
+#define PVHIP_COMPACT(K)                                                                                 \
+   do {                                                                                                  \
+      if (vec4 && iters == 1) K(4, 1);                                                                   \
+      else if (vec4) K(4, kCompactIters);                                                                \
+      else if (iters == 1) K(1, 1);                                                                      \
+      else K(1, kCompactIters);                                                                          \
+   } while (0)
+   PVHIP_COMPACT(PVHIP_COUNT);
    PVHIP_LAUNCHED("compact_count");
    hipLaunchKernelGGL(compact_scan_kernel, dim3(g.nbatch), dim3(1024), 0, (hipStream_t)stream,
          scratch, chunks, num_active);
    PVHIP_LAUNCHED("compact_scan");
-   if (vec4) {
-      hipLaunchKernelGGL(compact_write_kernel<4>, grid, dim3(kCompactThreads), 0, (hipStream_t)stream,
-            A, numExt, g.nf, scratch, chunks, entries, pos_start, numPos, num_active);
-   }
-   else {
-      hipLaunchKernelGGL(compact_write_kernel<1>, grid, dim3(kCompactThreads), 0, (hipStream_t)stream,
-            A, numExt, g.nf, scratch, chunks, entries, pos_start, numPos, num_active);
-   }
+   PVHIP_COMPACT(PVHIP_WRITE);
+#undef PVHIP_COMPACT
+#undef PVHIP_WRITE
+#undef PVHIP_COUNT
    PVHIP_LAUNCHED("compact_write");
    return PVHIP_OK;
 }

@@ -1890,9 +1890,15 @@ int cgemm_plan(const pvhip_recv_post_args *args, const PostParams &p, CGemmPlan 
       cs.splits = 1; // measured: the BF16 chunks do not gain from a split
    }
    else {
-      // ranges of at least 8 chunks, enough of them for about CGEMM_WG_TARGET workgroups
+      // ranges of at least two chunks, at most 8 of them (their partials are
+      // written and read back), for about CGEMM_WG_TARGET workgroups.  Shorter
+      // ranges than eight chunks pay on small grids, whose workgroups are
+      // otherwise too few to cover each other's staging: 8 images 32x32x256 ->
+      // 64x64x3 33.7 -> 28.6 us (8 ranges instead of 2), 4 x 24x24x256 ->
+      // 96x96x3 60.6 -> 27.5 us, 16 x 24x24x512 -> 48x48x1 51.4 -> 41.9 us (8
+      // instead of 4); large grids keep as many as before.
       long long sp = (CGEMM_WG_TARGET + blocks - 1) / blocks;
-      cs.splits    = (int)std::min<long long>(std::max<long long>(sp, 1), std::max(chunks / 8, 1));
+      cs.splits    = (int)std::min<long long>(std::max<long long>(sp, 1), std::min(8, std::max(chunks / 2, 1)));
    }
    cs.part      = nullptr;
    cs.nOut      = 0;

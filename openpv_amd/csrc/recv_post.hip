@@ -647,9 +647,24 @@ __device__ __forceinline__ void lca_epilogue_vthresh(
 
 // EPI: 0 GSyn only, 1 fused VTHRESH update, 2 fused update with either
 // transfer, 3 as 1 plus the active-list emission of full tiles.
-template <int ALIGN, int EPI, typename E = GatherBF16>
-__global__ void __launch_bounds__(256, E::WAVES) recv_post_mfma_bf16_kernel(
+//
+// FW: features per workgroup.  A wave reads every source fragment of the tile
+// from LDS, 1 KB for each FW / 64 MFMAs: with 64 features the four waves of a
+// workgroup ask for 256 bytes a cycle of the 128 a CU's LDS gives, with 128
+// (EPI 0, BF16 and FP8) for 128.  One 256x256x16 image -> 128x128x256, 12x12x16
+// patches, BF16: 34.7 -> 32.5 us; with one wave per SIMD the latency of the
+// fragment reads is what remains.
+template <int ALIGN, int EPI, typename E = GatherBF16, int FW = 64>
+__global__ void __launch_bounds__(256, FW == 64 ? E::WAVES : 2) recv_post_mfma_bf16_kernel(
       PostParams p, const typename E::T *Wb, int srcRowsMax, int srcColsMax, int Kpad) {
+   // features per workgroup and the epilogue layout that goes with them
+   constexpr int MF   = FW;
+   constexpr int MFB  = MF / 4 / 16;
+   constexpr int MOP  = MF + 4;
+   constexpr int MEQ  = MF / 4;
+   constexpr int MEPP = 256 / MEQ;
+   constexpr int MEP  = MTX * MTY / MEPP;
+   static_assert(FW == 64 || EPI == 0, "the fused epilogues are laid out for 64 features");
    using T = typename E::T;
    extern __shared__ float smem[];
    int const K       = p.nxp * p.nfp * p.nyp;
@@ -925,7 +940,9 @@ __global__ void __launch_bounds__(256, E::WAVES) recv_post_mfma_bf16_kernel(
    bool const fullTile = vec4 && fBase + MF <= p.post.nf && x0 + MTX <= p.post.nx
                          && y0 + MTY <= p.post.ny;
    if ((EPI == 1 || EPI == 3) && fullTile) {
-      lca_epilogue_vthresh<EPI == 3>(p, b, x0, y0, epr, eq, ef, outl + epr * MOP + 4 * eq, vpre);
+      if constexpr (FW == 64) {
+         lca_epilogue_vthresh<EPI == 3>(p, b, x0, y0, epr, eq, ef, outl + epr * MOP + 4 * eq, vpre);
+      }
       return;
    }
 #pragma unroll
@@ -2213,6 +2230,32 @@ int recv_post_launch(const pvhip_recv_post_args *args, PostParams &p, hipStream_
 #undef PVHIP_PERSIST_KS
 #undef PVHIP_PERSIST
          PVHIP_LAUNCHED("recv_post_mfma_persist");
+         return PVHIP_OK;
+      }
+      // 128 features per workgroup (half the LDS reads per MFMA; 34.7 -> 32.5 us
+      // on 256 workgroups) for a plain delivery whose grid still covers the chip
+      bool const wide = epi == 0 && !mfma32 && p.post.nf % 128 == 0 && align >= 2
+                        && (long long)tilesX * tilesY * (p.post.nf / 128) * p.post.nbatch >= 256;
+      if (wide) {
+         dim3 const wgrid(tilesX * tilesY, p.post.nf / 128, p.post.nbatch);
+         size_t const wlds = std::max(((size_t)srcRowsMax * pitch * esz + 3) / 4 * 4 + (size_t)Kpad * sizeof(int),
+                                      (size_t)MTX * MTY * (128 + 4) * sizeof(float));
+#define PVHIP_WIDE(AL)                                                                           \
+   do {                                                                                          \
+      if (fp8) {                                                                                 \
+         hipLaunchKernelGGL((recv_post_mfma_bf16_kernel<AL, 0, GatherFP8, 128>), wgrid, dim3(256), wlds, \
+               s, p, static_cast<const uint8_t *>(args->weights_lp), srcRowsMax, srcColsMax, Kpad); \
+      }                                                                                          \
+      else {                                                                                     \
+         hipLaunchKernelGGL((recv_post_mfma_bf16_kernel<AL, 0, GatherBF16, 128>), wgrid, dim3(256), wlds, \
+               s, p, static_cast<const __bf16 *>(args->weights_lp), srcRowsMax, srcColsMax, Kpad); \
+      }                                                                                          \
+   } while (0)
+         if (align == 8) PVHIP_WIDE(8);
+         else if (align == 4) PVHIP_WIDE(4);
+         else PVHIP_WIDE(2);
+#undef PVHIP_WIDE
+         PVHIP_LAUNCHED("recv_post_mfma_wide");
          return PVHIP_OK;
       }
 #define PVHIP_MFMA(AL, EP)                                                                       \

@@ -799,7 +799,9 @@ __global__ void __launch_bounds__(1024) recv_pre_cell_kernel(PreParams p, CellPl
                // (wy - cls) / t by the reciprocal, exact for these sizes
                w = ((int)((float)(nWy - cls) * c.invT + 0.5f) * c.qx + jx0) * (V * 4);
             };
-            constexpr int U = V <= 4 ? 8 : 4; // entries of a batch
+            // entries of a batch: few targets per thread leave registers for more
+            // in flight (two targets, 8 -> 16: 79 us of the small case -> 63)
+            constexpr int U = V <= 2 ? 16 : V <= 4 ? 8 : 4;
             uint4u en[U / 2];
             auto fetch = [&]() {
 #pragma unroll

@@ -1837,7 +1837,8 @@ int recv_post_launch(const pvhip_recv_post_args *args, PostParams &p, hipStream_
 // gives the launch about CGEMM_WG_TARGET workgroups (a workgroup runs its
 // channel chunks one after another, each staged through LDS, so a short
 // grid leaves the chip waiting on those loads).
-constexpr long long CGEMM_WG_TARGET = 2048;
+constexpr long long CGEMM_WG_TARGET  = 2048;
+constexpr long long CGEMM_SMALL_GRID = 600;
 
 struct CGemmPlan {
    CStrip cs;
@@ -1907,15 +1908,23 @@ int cgemm_plan(const pvhip_recv_post_args *args, const PostParams &p, CGemmPlan 
       cs.splits = 1; // measured: the BF16 chunks do not gain from a split
    }
    else {
-      // ranges of at least two chunks, at most 8 of them (their partials are
-      // written and read back), for about CGEMM_WG_TARGET workgroups.  Shorter
-      // ranges than eight chunks pay on small grids, whose workgroups are
-      // otherwise too few to cover each other's staging: 8 images 32x32x256 ->
-      // 64x64x3 33.7 -> 28.6 us (8 ranges instead of 2), 4 x 24x24x256 ->
-      // 96x96x3 60.6 -> 27.5 us, 16 x 24x24x512 -> 48x48x1 51.4 -> 41.9 us (8
-      // instead of 4); large grids keep as many as before.
+      // ranges of at least 8 chunks, enough of them for about CGEMM_WG_TARGET workgroups
       long long sp = (CGEMM_WG_TARGET + blocks - 1) / blocks;
-      cs.splits    = (int)std::min<long long>(std::max<long long>(sp, 1), std::min(8, std::max(chunks / 2, 1)));
+      cs.splits    = (int)std::min<long long>(std::max<long long>(sp, 1), std::max(chunks / 8, 1));
+      // A small grid takes shorter ranges, down to two chunks, up to about
+      // CGEMM_SMALL_GRID workgroups (two per CU; beyond, the partials cost more
+      // than the ranges save): 8 images 32x32x256 -> 64x64x3 34.0 (2 ranges) ->
+      // 28.7 us (8), 16 images 50.0 -> 41.1 (4), 4 x 24x24x256 -> 96x96x3 60.7 ->
+      // 27.5 (8), 44 x 33x8x256 -> 132x32x1 23.0 -> 22.1 (4).  Not where the
+      // weights leave room for one workgroup per CU: 8 x 24x24x128 -> 96x96x3
+      // with 16x16 patches, 91.2 (1) against 100.1 us (2).
+      if (lds <= 80 * 1024) {
+         int s = 8;
+         while (s > 1 && (s * blocks > CGEMM_SMALL_GRID || s > chunks / 2)) {
+            s /= 2;
+         }
+         cs.splits = std::max(cs.splits, s);
+      }
    }
    cs.part      = nullptr;
    cs.nOut      = 0;

@@ -550,7 +550,9 @@ int pvhip_ident_deliver(
  * extended (x,y) position p and pos_start[b][nPos] the count, so that
  * [pos_start[p], pos_start[p+1]) are the active features at p.  pos_start may
  * be NULL.  chunk_scratch is caller-owned device memory of
- * pvhip_active_compact_scratch_bytes(loc) bytes (no allocation inside). */
+ * pvhip_active_compact_scratch_bytes(loc) bytes (no allocation inside); that
+ * size never falls as the layer or its batch grows, so the scratch of a full
+ * batch serves a smaller one. */
 int pvhip_active_compact(
       const pvhip_loc *loc,
       const float *A,

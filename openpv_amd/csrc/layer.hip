@@ -7,6 +7,7 @@
 // operation (the library is built with -ffp-contract=off).
 #include "pvhip_internal.hpp"
 
+#include <algorithm>
 #include <mutex>
 
 namespace pvhip {
@@ -1006,9 +1007,16 @@ __global__ void __launch_bounds__(256) activity_to_bf16c_kernel(Geo g, const flo
 
 } // namespace
 
+// Room for either chunking, so that the size never falls as a layer or its
+// batch grows: scratch sized for a full batch also holds the (more numerous)
+// one-round counts of a smaller last one.  At most 4 * kSmallChunks bytes
+// beyond what the layer itself needs.
 size_t compact_scratch_bytes(const Geo &g) {
-   int const chunk = kCompactThreads * kCompactVec * compact_iters(g);
-   return (size_t)g.nbatch * (size_t)((g.numExt() + chunk - 1) / chunk) * sizeof(uint32_t);
+   auto chunks = [&](int iters) {
+      size_t const chunk = (size_t)kCompactThreads * kCompactVec * iters;
+      return (size_t)g.nbatch * (((size_t)g.numExt() + chunk - 1) / chunk);
+   };
+   return std::max(chunks(kCompactIters), std::min(chunks(1), (size_t)kSmallChunks)) * sizeof(uint32_t);
 }
 
 int active_from_segments(

@@ -105,6 +105,21 @@ def test_check_faults_is_exported_and_needs_a_device():
     assert abi.hip().pvhip_check_faults() in (0, 2)
 
 
+def test_active_list_scratch_of_a_full_batch_holds_for_a_smaller_one():
+    """pvhip_active_compact takes its chunk counts by a bare pointer: scratch
+    sized for a layer also serves the same layer with fewer batch elements or
+    rows, on both sides of the step between the two chunkings."""
+    H = abi.hip()
+    q = lambda *s: H.pvhip_active_compact_scratch_bytes(C.byref(abi.Loc.make(*s)))
+    for nx, nf, halo in ((32, 512, 2), (128, 512, 0), (5, 9, 1), (1, 1, 0)):
+        sizes = [q(nb, nx, 32, nf, halo) for nb in range(1, 80)]
+        assert sizes == sorted(sizes)
+        rows = [q(4, nx, ny, nf, halo) for ny in range(1, 300)]
+        assert rows == sorted(rows)
+    assert q(12, 32, 32, 512, 2) == 12 * 648 * 4          # one count per 1024 elements of a small layer
+    assert q(8192, 8, 8, 16, 0) == 8192 * 4 and q(20000, 8, 8, 16, 0) == 20000 * 4
+
+
 def test_channel_gemm_scratch_query_follows_the_launch_shape():
     """pvhip_recv_post_scratch_bytes (host logic only): the stride-4 transposed
     gather (32x32x512 -> 128x128x1) needs splits x GSyn floats of scratch:

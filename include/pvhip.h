@@ -285,8 +285,9 @@ typedef struct {
    /* Optional device scratch for the channel GEMM (FP32/BF16 forms with
     * several data patches per feature): the channels are split over
     * workgroups and their FP32 partial sums added in split order.  Size from
-    * pvhip_recv_post_scratch_bytes(args); NULL or smaller runs unsplit.  The
-    * library allocates nothing itself. */
+    * pvhip_recv_post_scratch_bytes(args); NULL runs unsplit, smaller runs the
+    * default number of ranges halved until it fits, or unsplit where
+    * cgemm_splits gives the number.  The library allocates nothing itself. */
    void *scratch;
    size_t scratch_bytes;
    /* Channel GEMM launch shape, 0 = the library's default: window starts per

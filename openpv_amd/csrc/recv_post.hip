@@ -2075,8 +2075,13 @@ int recv_post_launch(const pvhip_recv_post_args *args, PostParams &p, hipStream_
       if (st) {
          return st;
       }
-      if (pl.cs.splits > 1 && (!args->scratch || args->scratch_bytes < cgemm_scratch_bytes(p, pl))) {
-         pl.cs.splits = 1; // no room for the partials: one range of channels
+      // Without room for the partials an explicit number of ranges runs as one.
+      // The default number halves until they fit: a grid of fewer images takes
+      // more ranges, so scratch sized for a full batch may hold only half of
+      // those of a smaller one (32x32x256 -> 64x64x3: 17 images take 2, 16 take 4).
+      size_t const room = args->scratch ? args->scratch_bytes : 0;
+      while (pl.cs.splits > 1 && room < cgemm_scratch_bytes(p, pl)) {
+         pl.cs.splits = args->cgemm_splits > 0 ? 1 : pl.cs.splits / 2;
       }
       pl.cs.part = pl.cs.splits > 1 ? static_cast<float *>(args->scratch) : nullptr;
       pl.cs.nOut = (size_t)p.post.nbatch * p.post.numRes();

@@ -1914,12 +1914,12 @@ int cgemm_plan(const pvhip_recv_post_args *args, const PostParams &p, CGemmPlan 
       // A small grid takes shorter ranges, down to two chunks, up to about
       // CGEMM_SMALL_GRID workgroups (two per CU; beyond, the partials cost more
       // than the ranges save): 8 images 32x32x256 -> 64x64x3 34.0 (2 ranges) ->
-      // 31.0 us (4), 16 images 50.0 -> 41.1 (4), 4 x 24x24x256 -> 96x96x3 60.7 ->
-      // 37.9 (4), 44 x 33x8x256 -> 132x32x1 23.0 -> 22.1 (4).  Not where the
+      // 28.7 us (8), 16 images 50.0 -> 41.1 (4), 4 x 24x24x256 -> 96x96x3 60.7 ->
+      // 27.5 (8), 44 x 33x8x256 -> 132x32x1 23.0 -> 22.1 (4).  Not where the
       // weights leave room for one workgroup per CU: 8 x 24x24x128 -> 96x96x3
       // with 16x16 patches, 91.2 (1) against 100.1 us (2).
       if (lds <= 80 * 1024) {
-         int s = 4;
+         int s = 8;
          while (s > 1 && (s * blocks > CGEMM_SMALL_GRID || s > chunks / 2)) {
             s /= 2;
          }

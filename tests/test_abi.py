@@ -157,6 +157,33 @@ def test_channel_gemm_scratch_query_follows_the_launch_shape():
     assert q() == 0
 
 
+@pytest.mark.parametrize("shape,ranges", [
+    # images, nx, ny, nf of the source; scale, pre patch, features of the target
+    ((8, 32, 32, 256, 2, 8, 3), 8),      # 8 x 72 workgroups: under 600
+    ((9, 32, 32, 256, 2, 8, 3), 4),      # 8 x 81 is over it
+    ((16, 32, 32, 256, 2, 8, 3), 4),     # 4 x 144
+    ((17, 32, 32, 256, 2, 8, 3), 2),     # 4 x 153 is over; ranges of eight chunks
+    ((1, 16, 16, 128, 2, 8, 3), 4),      # 8 chunks: no range under two of them
+    ((4, 20, 20, 512, 2, 6, 3), 4),      # four ranges of eight chunks stay
+    ((1, 24, 24, 128, 4, 12, 3), 4),     # the weights leave room for two workgroups per CU
+    ((1, 24, 24, 128, 4, 16, 3), 1),     # they take more than 80 KB
+])
+def test_channel_gemm_default_ranges(shape, ranges):
+    """FP32's default number of channel ranges (host logic only), by its scratch."""
+    nb, nx, ny, nf, s, p, c = shape
+    stub = np.zeros(64, np.int32)
+    P = stub.ctypes.data_as(C.c_void_p)
+    a = abi.RecvPostArgs()
+    a.pre = abi.Loc.make(nb, nx, ny, nf, abi.host().pvhost_required_margin(nx, nx * s, p))
+    a.post = abi.Loc.make(nb, nx * s, ny * s, c, 0)
+    a.nxp = a.nyp = p // s
+    a.nfp, a.num_kernels_x, a.num_kernels_y = nf, s, s
+    a.start_x = a.start_y = a.kernel_x = a.kernel_y = a.inverse_x = a.inverse_y = P
+    a.window_nx, a.window_ny, a.dt_factor, a.arith = nx + 1, ny + 1, 1.0, abi.ARITH_FP32
+    gsyn = nb * nx * s * ny * s * c * 4
+    assert abi.hip().pvhip_recv_post_scratch_bytes(C.byref(a)) == (ranges * gsyn if ranges > 1 else 0)
+
+
 CASES = [
     ((1, 16, 16, 128, 2), (1, 32, 32, 3, 3), 8, 8),
     ((1, 32, 32, 512, 2), (1, 128, 128, 1, 6), 16, 16),

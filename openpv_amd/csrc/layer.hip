@@ -509,16 +509,22 @@ __global__ void __launch_bounds__(kRowThreads) error_update_vec_kernel(
 // 16-round ones fill it too, with a sixteenth of the counts to scan (and the
 // counts of pvhip_active_compact_noalloc's fixed workspace go as far as they
 // did).  One image of 256x256x16: the list and its sparse delivery 66.4 us with
-// 16 rounds, 47.1 us with one.
+// 16 rounds, 47.1 us with one.  The scan has one workgroup per image, whose
+// threads add up to kScanCounts counts each: the list of one image of
+// 128x128x448 (7 per thread) 30.8 us with 16 rounds, 22.1 with one, but of
+// 128x128x500 (8 per thread) 28.2 against 29.2.
 
 constexpr int kCompactThreads = 256;
 constexpr int kCompactIters   = 16;
 constexpr int kCompactVec     = 4; // elements per thread per iteration
 constexpr int kSmallChunks    = 8192;
+constexpr int kScanThreads    = 1024;
+constexpr int kScanCounts     = 7;
 
 inline int compact_iters(const Geo &g) {
-   int const one = kCompactThreads * kCompactVec;
-   return (long long)g.nbatch * ((g.numExt() + one - 1) / one) <= kSmallChunks ? 1 : kCompactIters;
+   int const one         = kCompactThreads * kCompactVec;
+   long long const image = (g.numExt() + one - 1) / one;
+   return image * g.nbatch <= kSmallChunks && image <= kScanThreads * kScanCounts ? 1 : kCompactIters;
 }
 
 // Loads elements [e, e+VEC) of one batch element's extended buffer (zeros past
@@ -579,11 +585,11 @@ __global__ void __launch_bounds__(kCompactThreads)
 }
 
 // One workgroup per batch element: exclusive scan of its chunk counts, in place.
-__global__ void __launch_bounds__(1024)
+__global__ void __launch_bounds__(kScanThreads)
       compact_scan_kernel(uint32_t *chunkCount, int chunksPerBatch, int64_t *numActive) {
    int const b        = blockIdx.x;
    uint32_t *c        = chunkCount + (size_t)b * chunksPerBatch;
-   __shared__ uint32_t partial[1024 / kWave];
+   __shared__ uint32_t partial[kScanThreads / kWave];
    int const per      = (chunksPerBatch + blockDim.x - 1) / blockDim.x;
    int const begin    = threadIdx.x * per;
    int const end      = min(begin + per, chunksPerBatch);
@@ -1024,7 +1030,7 @@ int active_from_segments(
       pvhip_sparse_entry *entries, int64_t *numActive, uint32_t *posStart, hipStream_t s) {
    PVHIP_REQUIRE(segW >= 1, "active list: segment width %d", segW);
    int const segsPerBatch = g.nx * g.ny * segsPerPos;
-   hipLaunchKernelGGL(compact_scan_kernel, dim3(g.nbatch), dim3(1024), 0, s, segCnt, segsPerBatch,
+   hipLaunchKernelGGL(compact_scan_kernel, dim3(g.nbatch), dim3(kScanThreads), 0, s, segCnt, segsPerBatch,
          numActive);
    PVHIP_LAUNCHED("compact_scan");
    int const segsPerBlock = 256 / kSegLanes;
@@ -1351,7 +1357,7 @@ int compact_launch(const pvhip_loc &l, const float *A, pvhip_sparse_entry *entri
    } while (0)
    PVHIP_COMPACT(PVHIP_COUNT);
    PVHIP_LAUNCHED("compact_count");
-   hipLaunchKernelGGL(compact_scan_kernel, dim3(g.nbatch), dim3(1024), 0, (hipStream_t)stream,
+   hipLaunchKernelGGL(compact_scan_kernel, dim3(g.nbatch), dim3(kScanThreads), 0, (hipStream_t)stream,
          scratch, chunks, num_active);
    PVHIP_LAUNCHED("compact_scan");
    PVHIP_COMPACT(PVHIP_WRITE);

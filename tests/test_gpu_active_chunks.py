@@ -1,6 +1,7 @@
 """The active list where its chunking changes: layers of one round per chunk up
-to the number of chunks that takes, the 16-round chunks beyond, several counts
-per thread of the scan, odd extended sizes, and empty and full buffers."""
+to the number of chunks that takes in one image and in the batch, the 16-round
+chunks beyond, several counts per thread of the scan, odd extended sizes, and
+empty and full buffers."""
 import numpy as np
 import pytest
 import torch
@@ -11,8 +12,11 @@ pytestmark = pytest.mark.gpu
 
 SHAPES = [  # nbatch, nx, ny, nf, halo; density
     ((1, 1, 1, 3, 0), 0.5), ((2, 13, 11, 7, 1), 0.3), ((5, 30, 20, 64, 2), 0.07),
-    ((1, 128, 128, 512, 0), 0.02),      # 8192 chunks of one round
-    ((1, 129, 128, 512, 0), 0.02),      # one more row: chunks of 16 rounds
+    ((1, 128, 128, 512, 0), 0.02), ((1, 129, 128, 512, 0), 0.02),
+    ((1, 128, 128, 448, 0), 0.02),      # 7168 chunks of one round, seven per thread of the scan
+    ((1, 129, 128, 448, 0), 0.02),      # one more column: chunks of 16 rounds
+    ((2, 128, 128, 256, 0), 0.02),      # 8192 in the batch
+    ((2, 129, 128, 256, 0), 0.02),      # ... and beyond
     ((2, 64, 64, 100, 0), 0.0), ((1, 64, 64, 100, 1), 1.0), ((300, 5, 5, 9, 1), 0.2),
 ]
 

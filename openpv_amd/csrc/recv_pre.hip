@@ -522,8 +522,8 @@ __global__ void __launch_bounds__(256) recv_pre_wave_kernel(PreParams p) {
 
 // ------------------------------------------------------------------ cell form
 //
-// Sparse source into a target t times finer along x and y with one data patch
-// per source feature (the reconstruction of an LCA column).  The t target
+// Sparse source into a target t >= 1 times finer along x and y with one data
+// patch per source feature (the reconstruction of an LCA column).  The t target
 // columns of one cell (first column congruent to the patch starts modulo t)
 // are covered by the same source columns, so the cw*nf targets of one thread
 // (cw columns of a cell, all features) walk the same entries of the active
@@ -551,12 +551,16 @@ __global__ void __launch_bounds__(256) recv_pre_wave_kernel(PreParams p) {
 // LDS.  Measured against recv_pre_lds_kernel, which stages the lists in LDS
 // between barriers: 64 images, 32x32x512 -> 128x128x1, 16x16 patches, 44,776
 // actives per image, 1368 -> 317 us; one image, 64x32x24 -> 128x64x1, 18x18
-// patches, 715 -> 79 us.
+// patches, 715 -> 63 us.  The other factors: t 1, 16 images 32x32x64 ->
+// 32x32x3, 3x3 patches, 5 % active, 73.6 -> 11.4 us; t 3, 16 images 32x32x128
+// -> 96x96x3, 9x9 patches, 7 % active, 240 -> 30.1; t 8, one image 32x32x256 ->
+// 256x256x1, 16x16 patches, 103 -> 20.1.
 struct CellPlan {
    int t, cw, qx, qy; // target cells per source cell; columns per thread; covering columns / rows
    int fstride;       // LDS floats of one feature: V * (qx*qy | 1)
    int splits;        // workgroups per (batch element, class)
    float invNf, invT; // 1 / pre.nf, 1 / t
+   float invQ, invQx; // 1 / (qx*qy), 1 / qx
 };
 
 // V consecutive LDS values at byte offset o from wl, a multiple of 4*V.
@@ -611,6 +615,9 @@ __global__ void __launch_bounds__(1024) recv_pre_cell_kernel(PreParams p, CellPl
    int const rho   = blockIdx.y % t;        // target rows rho, rho + t, ...
    int const dx0   = blockIdx.y / t * c.cw; // this workgroup's columns of a cell
    int const b     = blockIdx.z;
+   int const numPos     = nxExt * p.pre.nyExt();
+   const uint32_t *ps   = p.posStart + (size_t)b * ((size_t)numPos + 1);
+   uint32_t const total = ps[numPos]; // entries of this batch element
    // first column of cell 0 (at most 0) and the weight-row class of this residue
    // (from the first covered column and row; without one there is nothing to add)
    int X0 = 0, cls = 0;
@@ -635,24 +642,47 @@ __global__ void __launch_bounds__(1024) recv_pre_cell_kernel(PreParams p, CellPl
    int const waves = (items + kWave - 1) / kWave;
    int const first = (int)((long long)waves * blockIdx.x / c.splits) * kWave;
    int const last  = min((int)((long long)waves * (blockIdx.x + 1) / c.splits) * kWave, items);
-   {
+   if (total > 0) { // an empty list reads no weight
       // weights [f][jy][jx][V]: patch rows cls + t*jy, columns dx0 + t*jx ..
+      // SU pieces are loaded before the first is stored; a workgroup of one or
+      // two waves otherwise waits for each: 64 images 8x8x2048 -> 16x16x1 (82 KB
+      // of weights per workgroup of two waves) 58.4 -> 43.6 us at 5 % active, 32.8
+      // -> 6.1 for empty lists; 64 images 32x32x512 -> 128x128x1 274.8 -> 273.
+      constexpr int SU    = V <= 4 ? 8 : 4;
       int const q         = c.qx * c.qy;
       int const patchSize = p.nxp * p.nyp * nf;
-      for (int i = tid; i < nfPre * q; i += blockDim.x) {
-         int const f      = i / q;
-         int const j      = i - f * q;
-         int const jy     = j / c.qx;
-         int const jx     = j - jy * c.qx;
-         float const *src = p.W + (size_t)f * patchSize + ((cls + t * jy) * p.nxp + dx0 + t * jx) * nf;
-         float *dst       = wl + f * c.fstride + j * V;
+      int const pieces    = nfPre * q;
+      int const step      = blockDim.x;
+      for (int i0 = tid; i0 < pieces; i0 += SU * step) {
+         float w[SU][V];
+         int at[SU];
 #pragma unroll
-         for (int v = 0; v < V; v++) {
-            dst[v] = src[v];
+         for (int u = 0; u < SU; u++) {
+            int const i      = min(i0 + u * step, pieces - 1);
+            // quotients by the reciprocal, exact below 2^21 (the pieces are
+            // less than the LDS holds floats)
+            int const f      = (int)(((float)i + 0.5f) * c.invQ);
+            int const j      = i - f * q;
+            int const jy     = (int)(((float)j + 0.5f) * c.invQx);
+            int const jx     = j - jy * c.qx;
+            float const *src = p.W + (size_t)f * patchSize + ((cls + t * jy) * p.nxp + dx0 + t * jx) * nf;
+            at[u]            = f * c.fstride + j * V;
+#pragma unroll
+            for (int v = 0; v < V; v++) {
+               w[u][v] = src[v];
+            }
+         }
+#pragma unroll
+         for (int u = 0; u < SU; u++) {
+            if (i0 + u * step < pieces) {
+#pragma unroll
+               for (int v = 0; v < V; v++) {
+                  wl[at[u] + v] = w[u][v];
+               }
+            }
          }
       }
    }
-   const uint32_t *ps = p.posStart + (size_t)b * ((size_t)nxExt * p.pre.nyExt() + 1);
    const char *ent    = reinterpret_cast<const char *>(p.active + (size_t)b * p.pre.numExt());
    float *gb          = p.gsyn + (size_t)b * p.post.numRes();
    uint32_t const lastPair = (uint32_t)p.pre.numExt() - 2; // numExt is even
@@ -896,6 +926,8 @@ CellPlan cell_plan(const PreParams &p, size_t *lds) {
          c.cw    = cw;
          c.invNf = 1.0f / (float)p.pre.nf;
          c.invT  = 1.0f / (float)t;
+         c.invQ  = 1.0f / (float)(c.qx * c.qy);
+         c.invQx = 1.0f / (float)c.qx;
          return c;
       }
    }
@@ -965,9 +997,14 @@ int pvhip_recv_pre(const pvhip_recv_pre_args *a, pvhip_stream stream) {
       PVHIP_LAUNCHED("recv_pre_wave");
       return PVHIP_OK;
    }
-   // Cell form for a sparse source into a finer, narrow target (1368 -> 317 us
-   // and 715 -> 79 us against the LDS-staged form below, which keeps coarser
-   // targets, several data patches and weights too large for the LDS).
+   // Cell form for a sparse source into a narrow target as fine or finer, t from
+   // 1 to 8, densities from 0 to 100 %: 3 to 23 times as fast as the LDS-staged
+   // form below at each of 25 geometries (the closest 44.2 against 14.7 us for 64
+   // images 16x16x64 -> 32x32x8), and than the per-neuron form where that one has
+   // no room (many features, few columns): 128 against 44.8 us for 64 images
+   // 16x16x1024 -> 16x16x1 at 5 %, 31 against 28 for 64 images 8x8x2048 ->
+   // 16x16x1 at 0.5 %, equal for empty lists.  Coarser targets, several data
+   // patches and weights too large for the LDS keep those.
    size_t cellLds      = 0;
    CellPlan cp         = cell_plan(p, &cellLds);
    if (cp.t > 0) {

@@ -652,7 +652,7 @@ __device__ __forceinline__ void lca_epilogue_vthresh(
 // from LDS, 1 KB for each FW / 64 MFMAs: with 64 features the four waves of a
 // workgroup ask for 256 bytes a cycle of the 128 a CU's LDS gives, with 128
 // (EPI 0, BF16 and FP8) for 128.  One 256x256x16 image -> 128x128x256, 12x12x16
-// patches, BF16: 34.7 -> 32.5 us; with one wave per SIMD the latency of the
+// patches, BF16: 34.4 -> 32.0 us; with one wave per SIMD the latency of the
 // fragment reads is what remains.
 template <int ALIGN, int EPI, typename E = GatherBF16, int FW = 64>
 __global__ void __launch_bounds__(256, FW == 64 ? E::WAVES : 2) recv_post_mfma_bf16_kernel(
@@ -2251,26 +2251,48 @@ int recv_post_launch(const pvhip_recv_post_args *args, PostParams &p, hipStream_
          PVHIP_LAUNCHED("recv_post_mfma_persist");
          return PVHIP_OK;
       }
-      // 128 features per workgroup (half the LDS reads per MFMA; 34.7 -> 32.5 us
-      // on 256 workgroups) for a plain delivery whose grid still covers the chip
-      bool const wide = epi == 0 && !mfma32 && p.post.nf % 128 == 0 && align >= 2
-                        && (long long)tilesX * tilesY * (p.post.nf / 128) * p.post.nbatch >= 256;
+      // 128 features per workgroup (half the LDS reads per MFMA) for a plain
+      // delivery whose grid still covers the chip.  Measured against 64 on grids
+      // of 256 to 2048 workgroups (us of 64 -> of 128 features):
+      //  * 2-aligned windows read a fragment in four pieces, which collide on the
+      //    banks where the starts are more than two values apart.  FP8: K 64 12.1
+      //    -> 11.9 (384 workgroups, one and a half per CU: 14.7 against 14.9), K
+      //    192 20.2 -> 16.6, K 768 51.9 -> 32.9.  BF16: K 192 27.1 -> 26.1 (384:
+      //    13.4 against 13.5), K 320 13.7 -> 13.3, K 768 21.0 -> 17.9, K 1280 29.4
+      //    -> 23.7; starts two apart, K 256 10.8 against 11.5, K 576 15.3 -> 14.9.
+      //  * Wider reads, FP8: 64 features are faster, K 2304 30.6 against 39.2, K
+      //    256 47.3 against 56.6, K 128 9.6 against 11.9.
+      //  * Wider reads, BF16: long patches gain, K 2304 34.4 -> 32.0, K 1024 21.5 ->
+      //    20.3, K 800 17.4 -> 16.7, and K 576 where starts 32 or more values apart
+      //    meet on the same banks (17.3 -> 16.8).  Shorter ones are bound by staging
+      //    and stores, which two workgroups per CU cover less well than four: K 512
+      //    13.5 against 13.9, K 256 45.3 against 48.5, K 32 29.8 against 33.3.
+      //    A half-empty last round costs twice as much with twice the features, so
+      //    only where the 64-feature grid takes an even number of rounds of 256
+      //    (K 1024, 384 workgroups 27.4 against 28.9, 512 workgroups 32.7 -> 30.4).
+      long long const wideGrid = (long long)tilesX * tilesY * (p.post.nf / 128) * p.post.nbatch;
+      bool const even          = (2 * wideGrid + 255) / 256 % 2 == 0;
+      bool wide                = epi == 0 && !mfma32 && p.post.nf % 128 == 0 && wideGrid >= 256;
+      if (align == 2) {
+         int const any  = fp8 ? 192 : (step > 2 ? 320 : 1 << 30); // K taken whatever the rounds
+         int const some = fp8 ? 64 : (step > 2 ? 192 : 576);      // ... with an even number
+         wide           = wide && K >= (even ? some : any);
+      }
+      else {
+         wide = wide && !fp8 && align > 2 && even && (K >= 768 || (K >= 576 && step >= 32));
+      }
       if (wide) {
          dim3 const wgrid(tilesX * tilesY, p.post.nf / 128, p.post.nbatch);
          size_t const wlds = std::max(((size_t)srcRowsMax * pitch * esz + 3) / 4 * 4 + (size_t)Kpad * sizeof(int),
                                       (size_t)MTX * MTY * (128 + 4) * sizeof(float));
 #define PVHIP_WIDE(AL)                                                                           \
-   do {                                                                                          \
-      if (fp8) {                                                                                 \
-         hipLaunchKernelGGL((recv_post_mfma_bf16_kernel<AL, 0, GatherFP8, 128>), wgrid, dim3(256), wlds, \
-               s, p, static_cast<const uint8_t *>(args->weights_lp), srcRowsMax, srcColsMax, Kpad); \
-      }                                                                                          \
-      else {                                                                                     \
-         hipLaunchKernelGGL((recv_post_mfma_bf16_kernel<AL, 0, GatherBF16, 128>), wgrid, dim3(256), wlds, \
-               s, p, static_cast<const __bf16 *>(args->weights_lp), srcRowsMax, srcColsMax, Kpad); \
-      }                                                                                          \
-   } while (0)
-         if (align == 8) PVHIP_WIDE(8);
+   hipLaunchKernelGGL((recv_post_mfma_bf16_kernel<AL, 0, GatherBF16, 128>), wgrid, dim3(256), wlds, \
+         s, p, static_cast<const __bf16 *>(args->weights_lp), srcRowsMax, srcColsMax, Kpad)
+         if (fp8) {
+            hipLaunchKernelGGL((recv_post_mfma_bf16_kernel<2, 0, GatherFP8, 128>), wgrid, dim3(256), wlds, s, p,
+                  static_cast<const uint8_t *>(args->weights_lp), srcRowsMax, srcColsMax, Kpad);
+         }
+         else if (align == 8) PVHIP_WIDE(8);
          else if (align == 4) PVHIP_WIDE(4);
          else PVHIP_WIDE(2);
 #undef PVHIP_WIDE

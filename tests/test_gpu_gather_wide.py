@@ -1,7 +1,8 @@
 """The plain delivery with 128 features per workgroup (BF16, FP8) against the
 oracle's gather: every alignment class of its LDS reads, patches with and
 without a padded last k-step, ragged position tiles, accumulate, and the
-geometries beside it (too few workgroups, features not a multiple of 128).
+geometries beside it that keep 64 features (short patches, too few workgroups,
+an odd number of rounds of them, features not a multiple of 128).
 Operands are small integers times powers of two, exact in both formats, whose
 products and sums are exact in FP32 too: the results are equal."""
 import numpy as np
@@ -22,6 +23,16 @@ CASES = [
     ((64, 34, 34, 3, 4), (64, 17, 17, 128, 0), 8),    # 2-aligned, rows of 24 values
     ((1, 32, 32, 8, 4), (1, 16, 16, 256, 0), 8),      # too few workgroups
     ((16, 64, 64, 8, 4), (16, 32, 32, 192, 0), 8),    # not a multiple of 128
+    ((16, 64, 64, 8, 4), (16, 32, 32, 256, 0), 10),   # 8-aligned, K 800: BF16 takes 128
+    ((16, 64, 64, 12, 4), (16, 32, 32, 256, 0), 10),  # ... K 1200: half of the last k-step is padding
+    ((2, 32, 32, 4, 2), (2, 16, 16, 128, 0), 6),      # 64 features, K 144: a padded last k-step
+    ((64, 64, 64, 3, 6), (64, 16, 16, 256, 0), 16),   # 4-aligned, K 768, stride 4: BF16 takes 128
+    ((40, 36, 34, 1, 12), (40, 18, 17, 256, 0), 24),  # 2-aligned, K 576, ragged: both take 128, 480 workgroups
+    ((24, 64, 64, 5, 4), (24, 32, 32, 256, 0), 8),    # 2-aligned, K 320, 384 workgroups: both take 128
+    ((17, 36, 36, 16, 2), (17, 18, 18, 384, 0), 6),   # starts 32 values apart, K 576, 306 workgroups: 64
+    ((64, 32, 32, 16, 2), (64, 16, 16, 256, 0), 6),   # ... with 256: BF16 takes 128
+    ((64, 36, 36, 1, 4), (64, 18, 18, 128, 0), 8),    # 2-aligned, K 64, 384 workgroups: 64
+    ((64, 32, 32, 1, 4), (64, 16, 16, 256, 0), 8),    # ... with 256: FP8 takes 128
 ]
 
 

@@ -20,8 +20,15 @@ CASES = [
     ((1, 4, 37, 8, 1), (1, 8, 74, 3, 2), 6, 5),        # ... along y only
     ((2, 12, 10, 130, 2), (2, 24, 20, 3, 3), 8, 0),    # two feature blocks and a ragged one
     ((1, 9, 9, 40, 2), (1, 36, 36, 2, 6), 16, 3),      # two item blocks
-    ((1, 140, 6, 16, 1), (1, 280, 12, 1, 1), 4, 0),    # columns past the prefetched ones
+    ((1, 140, 6, 16, 1), (1, 280, 12, 1, 1), 4, 0),    # several 32-column steps a row
     ((3, 6, 6, 20, 1), (3, 6, 6, 2, 1), 3, 7),         # one to one
+    # post rows longer than the 768 elements whose loads are issued a row ahead,
+    # windows of over 80 KB (a ring of nyp rows, two barriers a row), chunks that
+    # walk several pre rows and cross from one image to the next
+    ((2, 64, 4, 20, 2), (2, 256, 16, 3, 6), 16, 5),
+    ((2, 20, 5, 16, 1), (2, 160, 40, 3, 8), 24, 100),  # eight new post rows a pre row
+    # eight new post rows where the ring has room for them, and fewer than 256 elements each
+    ((2, 5, 7, 70, 1), (2, 40, 56, 1, 4), 16, 6),
 ]
 
 

@@ -1,8 +1,10 @@
 """The 16-byte forms of the layer updates and of the transfer give the bits of
 the element-wise forms (which the oracle tests pin): the same call on buffers
-one value off the 16-byte boundary runs those.  One quad in all, layers that
-end inside a workgroup, one and several channels, A(t-1) read and recomputed,
-the chunked BF16 copy, and A left out."""
+one value off the 16-byte boundary runs those.  Images at the 1024 neurons the
+16-byte form starts at (smaller ones are element-wise either way) and layers
+that end inside a workgroup, one and several channels, A(t-1) read and
+recomputed (for ISTA from 2^18 neurons on), the chunked BF16 copy, and A left
+out."""
 import numpy as np
 import pytest
 import torch
@@ -11,7 +13,9 @@ from openpv_amd import abi, runtime as R
 
 pytestmark = pytest.mark.gpu
 FMAX = float(np.finfo(np.float32).max)
-SHAPES = [(1, 1, 1, 4, 0), (2, 5, 3, 12, 1), (3, 16, 9, 64, 2), (1, 6, 2, 2, 2), (2, 33, 17, 32, 3)]
+SHAPES = [(1, 1, 1, 4, 0), (2, 5, 3, 12, 1), (3, 16, 9, 64, 2), (1, 6, 2, 2, 2), (2, 33, 17, 32, 3),
+          (2, 16, 16, 4, 0), (1, 6, 171, 2, 2), (3, 7, 37, 4, 0), (2, 43, 19, 12, 1), (1, 17, 15, 4, 2),
+          (2, 64, 57, 36, 1)]
 
 
 def at(x, off):

@@ -1911,20 +1911,21 @@ int cgemm_plan(const pvhip_recv_post_args *args, const PostParams &p, CGemmPlan 
       // ranges of at least 8 chunks, enough of them for about CGEMM_WG_TARGET workgroups
       long long sp = (CGEMM_WG_TARGET + blocks - 1) / blocks;
       cs.splits    = (int)std::min<long long>(std::max<long long>(sp, 1), std::max(chunks / 8, 1));
-      // A small grid takes up to 8 shorter ranges, of two chunks or more, up to
-      // about CGEMM_SMALL_GRID workgroups (two per CU; beyond, the partials cost
-      // more than the ranges save): 8 images 32x32x256 -> 64x64x3 34.1 us (2
-      // ranges), 30.4 (4), 27.8 (8); 16 images 49.0 (2), 39.9 (4), 42.3 (8);
-      // 4 x 24x24x256 -> 96x96x3 32.0 (2), 22.8 (4), 19.9 (8), with 12x12
-      // patches, 2 images, 60.8, 37.2, 25.8; 44 x 33x8x256 -> 132x32x1 22.6 (2),
-      // 21.3 (4).  Not where the weights leave room for one workgroup per CU:
-      // 8 x 24x24x128 -> 96x96x3 with 16x16 patches, 91.1 (1) against 99.4 us (2).
-      // Where ranges of eight chunks already are four, that number stays: it
-      // is the one callers size the scratch of a 512-feature source by (8 would
-      // take 25.1 us instead of 25.7 for 16 x 20x20x512 -> 40x40x3, 18.6 instead
-      // of 25.3 for 4).
-      if (lds <= 80 * 1024 && cs.splits < 4) {
-         int s = 8;
+      // A small grid takes up to four shorter ranges, of two chunks or more, up
+      // to about CGEMM_SMALL_GRID workgroups (two per CU; beyond, the partials
+      // cost more than the ranges save): 8 images 32x32x256 -> 64x64x3 34.1 us (2
+      // ranges), 30.4 (4); 16 images 49.0 (2), 39.9 (4), 42.3 (8); 4 x 24x24x256 ->
+      // 96x96x3 32.0 (2), 22.8 (4), with 12x12 patches, 2 images, 60.8, 37.2; 44 x
+      // 33x8x256 -> 132x32x1 22.6 (2), 21.3 (4).  Not where the weights leave room
+      // for one workgroup per CU: 8 x 24x24x128 -> 96x96x3 with 16x16 patches, 91.1
+      // (1) against 99.4 us (2).
+      // Eight ranges would be faster on the smallest grids (27.8 us for the first,
+      // 19.9 and 25.8 for the third pair) but regroup the sums once more, which a
+      // hard threshold behind them amplifies: over 24 inputs the adjoint's
+      // gradients came out up to 3.5 times as far from 64 bits as with four on
+      // three, and nearer on three others.
+      if (lds <= 80 * 1024) {
+         int s = 4;
          while (s > 1 && (s * blocks > CGEMM_SMALL_GRID || s > chunks / 2)) {
             s /= 2;
          }

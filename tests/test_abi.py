@@ -159,12 +159,12 @@ def test_channel_gemm_scratch_query_follows_the_launch_shape():
 
 @pytest.mark.parametrize("shape,ranges", [
     # images, nx, ny, nf of the source; scale, pre patch, features of the target
-    ((8, 32, 32, 256, 2, 8, 3), 8),      # 8 x 72 workgroups: under 600
-    ((9, 32, 32, 256, 2, 8, 3), 4),      # 8 x 81 is over it
-    ((16, 32, 32, 256, 2, 8, 3), 4),     # 4 x 144
+    ((8, 32, 32, 256, 2, 8, 3), 4),      # four at most
+    ((16, 32, 32, 256, 2, 8, 3), 4),     # 4 x 144 workgroups: under 600
     ((17, 32, 32, 256, 2, 8, 3), 2),     # 4 x 153 is over; ranges of eight chunks
-    ((1, 16, 16, 128, 2, 8, 3), 4),      # 8 chunks: no range under two of them
-    ((4, 20, 20, 512, 2, 6, 3), 4),      # four ranges of eight chunks stay
+    ((1, 16, 16, 128, 2, 8, 3), 4),      # 8 chunks: ranges of two
+    ((1, 16, 16, 64, 2, 8, 3), 2),       # 4 chunks: no range under two of them
+    ((4, 20, 20, 512, 2, 6, 3), 4),      # four ranges of eight chunks
     ((1, 24, 24, 128, 4, 12, 3), 4),     # the weights leave room for two workgroups per CU
     ((1, 24, 24, 128, 4, 16, 3), 1),     # they take more than 80 KB
 ])

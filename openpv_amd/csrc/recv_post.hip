@@ -2339,8 +2339,12 @@ int recv_post_launch(const pvhip_recv_post_args *args, PostParams &p, hipStream_
       int const tilesX     = (p.post.nx + TX - 1) / TX;
       int const tilesY     = (p.post.ny + TY - 1) / TY;
       // 64 features per workgroup (more products per LDS read), 32 where 64
-      // would be half padding or the grid would leave CUs idle: four steps of one
-      // image 128x64x1 -> 64x32x24, 18x18 patches (32 workgroups), 798 -> 695 us
+      // would be half padding or the grid would leave CUs idle: 1.5 to 1.9 times as
+      // fast at each of 23 shapes of 32 to 224 workgroups (224 of 7 images
+      // 128x64x1 -> 64x32x64, 18x18 patches, 63.6 -> 40.5 us; 128 of one image
+      // 128x128x16 -> 64x64x64, 12x12, 346 -> 181); the line lies at one
+      // workgroup per CU.  (32 features stay ahead a little further: 256 workgroups
+      // 65.1 against 39.2 us, 512 62.0 against 56.9, 768 74.2 against 75.9.)
       bool const narrow = p.post.nf <= 32
                           || (long long)tilesX * tilesY * ((p.post.nf + 63) / 64) * p.post.nbatch < 256;
       for (int FB : {64, 32}) {
